@@ -112,7 +112,7 @@ def draw(rng):
                      delta=1e-5, coupling=0.1, tol=1e-8, lanes=rng.choice([0, 1]))
         else:
             c = dict(kind="inel", n=_logint(rng, 16, 64), nbl=_logint(rng, 4, 10), nE=_logint(rng, 40, 160),
-                     nk=rng.choice([1, 2, 3]), delta=1e-5, passes=rng.choice([5, 8, 10]),
+                     nk=rng.choice([2, 3]), delta=1e-5, passes=rng.choice([5, 8, 10]),
                      lanes=rng.choice([0, 1]))
         items = c.get("nE", c.get("npts", 1)) * c.get("nk", 1)
         blocks = 16.0 * c["n"] ** 2 * c["nbl"] * items
@@ -187,6 +187,12 @@ def _slab(n, nbl, seed, nk=1, mirror=True, side=False):
     return out
 
 
+# Centre of the bias window of the SCBA cases: off the band centre, where the
+# layers of a clean lead of odd width have a zero eigenvalue and E = 0 on the
+# grid makes every evaluation ill-conditioned.
+_MU0 = 0.0137
+
+
 def _fermi(E, mu, kT):
     return 1.0 / (1.0 + np.exp(np.clip((E - mu) / kT, -500.0, 500.0)))
 
@@ -199,7 +205,7 @@ def _inputs(case, seed):
     x = {}
     if k == "T" and case["model"] == "ribbon":
         s = [_ribbon(n, nbl, 0.5 if n >= 32 else 0.1, seed, weak_lead=not case["mirror"])]
-        E = energy_grid(case["nE"], -3.5, 3.5)
+        E = energy_grid(case["nE"], -3.5, 3.47)  # off E = 0: see _MU0
     elif k in ("T", "multi", "ldos"):
         s = _slab(n, nbl, seed, case.get("nk", 1), case.get("mirror", True), side=(k == "multi"))
         E = energy_grid(case["nE"], -2.0, 2.0)
@@ -228,9 +234,9 @@ def _inputs(case, seed):
             x["frm"] = np.stack([_fermi(E, bias / 2, kT), _fermi(E, -bias / 2, kT), np.zeros(m)], axis=1)
         return s, x
     kT, bias = KB_EV * 300.0, 0.2
-    E = energy_grid(case["nE"], -bias / 2 - 10 * kT, bias / 2 + 10 * kT)
+    E = energy_grid(case["nE"], _MU0 - bias / 2 - 10 * kT, _MU0 + bias / 2 + 10 * kT)
     x["E"] = E
-    x["frm"] = np.stack([_fermi(E, bias / 2, kT), _fermi(E, -bias / 2, kT), np.zeros_like(E)], axis=1)
+    x["frm"] = np.stack([_fermi(E, _MU0 + bias / 2, kT), _fermi(E, _MU0 - bias / 2, kT), np.zeros_like(E)], axis=1)
     if k == "scba":
         s = [_ribbon(n, nbl, 0.2, seed)]
         x["coupling"] = np.full(n * nbl, case["coupling"])
@@ -309,11 +315,11 @@ def tolerance(case):
     """Relative bars from FP64 runs against ``exact`` over several seeds: the
     blocks E S - H - Sigma at real E have condition numbers up to 1/eta, so a
     few energies of each grid carry most of the difference and it varies by a
-    factor of 30 from seed to seed (T: 4e-9 .. 2e-7; SCBA: 2e-7, its own
-    stopping tolerance; contour points are well conditioned).  ``differ``:
+    factor of 30 from seed to seed (T: 4e-9 .. 2e-7; SCBA: 2e-8 .. 3e-6, its own
+    stopping tolerance amplified; contour points are well conditioned).  ``differ``:
     decimation and SCBA counts whose test value falls on the threshold."""
     rel = {"T": 2e-6 if case["n"] >= 32 else 1e-7, "multi": 2e-7, "ldos": 2e-7, "dm0": 1e-12, "dm1": 2e-7,
-           "scba": 2e-6, "inel": 5e-8}[case["kind"]]
+           "scba": 2e-5, "inel": 5e-8}[case["kind"]]
     return {"rel": rel, "differ": 0.02}
 
 
@@ -352,7 +358,8 @@ class _Dev:
 
 
 def _inv(a):
-    return torch.linalg.inv(a.contiguous())
+    # in parts: the batched LU's workspace grows with batch * order
+    return torch.cat([torch.linalg.inv(p.contiguous()) for p in a.split(max(1, 8192 // a.shape[-1]))])
 
 
 def _surface(dev, c, z):
@@ -567,8 +574,8 @@ def _exact_inel(case, s, x):
     for _ in range(case["passes"]):
         cur = torch.zeros(nk * ne, 2, dtype=torch.float64, device="cuda")
         Gr, Gn = torch.empty_like(A0), torch.empty_like(A0)
-        for a in range(0, nk * ne, 64):
-            b = slice(a, min(a + 64, nk * ne))
+        for a in range(0, nk * ne, 32):
+            b = slice(a, min(a + 32, nk * ne))
             G = _inv(A0[b] - Sr[b] if Sr is not None else A0[b])
             Gr[b] = G
             Gn[b] = G @ (S0[b] + Sn[b] if Sn is not None else S0[b]) @ _dag(G)
