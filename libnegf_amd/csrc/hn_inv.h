@@ -6,7 +6,7 @@ namespace hn {
 
 constexpr int kInvSuper = 64;  // max super-panel width: deferred rank-64 updates
 
-// Largest n handled by the single-workgroup LDS kernel.
+// Largest n handled by the one-workgroup LU kernel (no workspace needed).
 int inv_lds_max_n(int real_bytes);
 
 // Workspace of the blocked path, for `batch` items of order n.

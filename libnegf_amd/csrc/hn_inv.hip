@@ -3,9 +3,9 @@
 // Replaces zinv (ZGETRF + ZGETRS against I, inversions.F90:807-839) and
 // cu_Zinverse (gpuroutines.cu:449-523) for whole batches of blocks.
 //
-// Small blocks (n^2 complex fit in LDS): one workgroup per block runs an
-// in-place Gauss-Jordan elimination with partial pivoting entirely in LDS,
-// followed by the column interchanges that undo the row pivoting.
+// Blocks up to 96 (FP32: 128): one workgroup per block, LU with partial pivoting
+// and the substitutions in registers, on the matrix cores (k_lu_inv_mx; FP64 up
+// to 16 on a thread grid, k_lu_inv_2d).
 //
 // Large blocks (up to n = 1024): in-place Gauss-Jordan with lazy pivoting on
 // the row-major view M = A^T, so that rows of M are contiguous columns of A
@@ -28,7 +28,6 @@ namespace hn {
 namespace {
 
 constexpr int NT = 256;
-constexpr int kLdsBudget = 160 * 1024 - 2048;
 
 template <typename R> struct CT_;
 template <> struct CT_<double> { typedef double2 t; };
@@ -53,98 +52,6 @@ template <typename C> __device__ inline C crecip(C b) {
 }
 template <typename C> __device__ inline auto cabs1(C a) -> decltype(a.x) {
   return fabs(a.x) + fabs(a.y);
-}
-
-// wave-level argmax of (v, i): larger v wins, ties -> smaller index
-template <typename R> __device__ inline void wave_argmax(R &v, int &i) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    R ov = __shfl_xor(v, off);
-    int oi = __shfl_xor(i, off);
-    if (ov > v || (ov == v && oi >= 0 && (i < 0 || oi < i))) {
-      v = ov;
-      i = oi;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// single-workgroup LDS Gauss-Jordan
-// ---------------------------------------------------------------------------
-template <typename R>
-__global__ __launch_bounds__(NT) void k_inv_lds(int n, typename CT_<R>::t *A, long long sA,
-                                                typename CT_<R>::t *Ainv, long long sAinv,
-                                                const int *active, int *status) {
-  typedef typename CT_<R>::t C;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int b = blockIdx.x;
-  if (active && active[b] == 0) return;
-  C *M = (C *)smem;
-  C *rowbuf = M + (size_t)n * n;
-  C *colbuf = rowbuf + n;
-  int *perm = (int *)(colbuf + n);
-  __shared__ int s_p, s_sing;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const C *Ab = A + (long long)b * sA;
-  for (int e = tid; e < n * n; e += NT) M[e] = Ab[e];
-  if (tid == 0) s_sing = 0;
-  // 2-D thread mapping for the rank-1 update: thread -> (row i, column phase)
-  const int cpar = NT / n;  // n <= NT here
-  const int ui = tid % n, uj0 = tid / n;
-  const bool upd = uj0 < cpar;
-  __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    if (wave == 0) {
-      R best = R(-1);
-      int bi = -1;
-      for (int i = k + lane; i < n; i += 64) {
-        R v = cabs1(M[i + (size_t)k * n]);
-        if (v > best) { best = v; bi = i; }
-      }
-      wave_argmax(best, bi);
-      if (lane == 0) {
-        s_p = bi < 0 ? k : bi;
-        if (!(best > R(0))) s_sing = 1;
-      }
-    }
-    __syncthreads();
-    const int p = s_p;
-    if (p != k)
-      for (int j = tid; j < n; j += NT) {
-        C t = M[k + (size_t)j * n];
-        M[k + (size_t)j * n] = M[p + (size_t)j * n];
-        M[p + (size_t)j * n] = t;
-      }
-    if (tid == 0) perm[k] = p;
-    __syncthreads();
-    const C pinv = crecip(M[k + (size_t)k * n]);
-    for (int j = tid; j < n; j += NT) rowbuf[j] = (j == k) ? pinv : cmul(M[k + (size_t)j * n], pinv);
-    for (int i = tid; i < n; i += NT) colbuf[i] = (i == k) ? C{0, 0} : M[i + (size_t)k * n];
-    __syncthreads();
-    if (upd) {
-      const C ci = colbuf[ui];
-      for (int j = uj0; j < n; j += cpar) {
-        size_t e = ui + (size_t)j * n;
-        if (ui == k) M[e] = rowbuf[j];
-        else if (j == k) M[e] = cneg(cmul(ci, pinv));
-        else M[e] = csub(M[e], cmul(ci, rowbuf[j]));
-      }
-    }
-    __syncthreads();
-  }
-  for (int k = n - 1; k >= 0; --k) {
-    const int p = perm[k];
-    if (p != k)
-      for (int i = tid; i < n; i += NT) {
-        C t = M[i + (size_t)k * n];
-        M[i + (size_t)k * n] = M[i + (size_t)p * n];
-        M[i + (size_t)p * n] = t;
-      }
-    __syncthreads();
-  }
-  C *Ob = Ainv + (long long)b * sAinv;
-  for (int e = tid; e < n * n; e += NT) Ob[e] = M[e];
-  if (tid == 0 && s_sing && status) atomicOr(&status[b], (int)ST_SINGULAR);
 }
 
 // ---------------------------------------------------------------------------
@@ -223,7 +130,7 @@ __device__ inline unsigned wave_min32(unsigned k) {
 }
 
 // ---------------------------------------------------------------------------
-// LU inverse of blocks up to 64 (complex double), one workgroup per block
+// LU inverse of blocks up to 16 (complex double), one workgroup per block
 // ---------------------------------------------------------------------------
 // The reference's algorithm: ZGETRF (partial pivoting; the pivot is the first
 // largest |Re| + |Im| of the column in the current row order, as IZAMAX
@@ -299,10 +206,11 @@ __device__ inline double2 fms_c(double2 x, double2 m, double2 y) {
   x.y = fma(-m.y, y.x, x.y);
   return x;
 }
-// value `v` of lane `src` (lane index within the wave), for every lane
+
+// value `v` of the lane at byte index `src` (4 x lane) within the wave, for every lane
 __device__ inline double bperm(double v, int src) {
-  const int lo = __builtin_amdgcn_ds_bpermute(src << 2, __double2loint(v));
-  const int hi = __builtin_amdgcn_ds_bpermute(src << 2, __double2hiint(v));
+  const int lo = __builtin_amdgcn_ds_bpermute(src, __double2loint(v));
+  const int hi = __builtin_amdgcn_ds_bpermute(src, __double2hiint(v));
   return __hiloint2double(hi, lo);
 }
 __device__ inline double2 bperm(double2 v, int src) {
@@ -435,7 +343,7 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
       // that holds it (same wave)
       const int ps = __builtin_amdgcn_readfirstlane(pi);
       static_for<TB>([&](auto J) {
-        const C u = bperm(pick0<TB, J>(B.v, ps), gbase + prb);
+        const C u = bperm(pick0<TB, J>(B.v, ps), (gbase + prb) << 2);
         static_for<TB>([&](auto I) { B.v[I][J] = fms_c(B.v[I][J], m[I], u); });
       });
       if (k + 1 < n)
@@ -457,7 +365,7 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
       coef[T] = (B.pos[T] < i) ? Ut[utri(B.pos[T], i)] : C{0, 0};
     });
     static_for<TB>([&](auto J) {
-      const C xq = bperm(cmul(pick0<TB, J>(B.v, qs), uinv), gbase + qrb);
+      const C xq = bperm(cmul(pick0<TB, J>(B.v, qs), uinv), (gbase + qrb) << 2);
       // coef = 0 on row q and below position i
       static_for<TB>([&](auto T) { B.v[T][J] = fms_c(B.v[T][J], coef[T], xq); });
     });
@@ -477,6 +385,470 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
       const int pc = s_perm[c];
       static_for<TB>([&](auto I) {
         if (rb * TB + I < n) Ob[B.pos[I] + (size_t)pc * n] = B.v[I][J];
+      });
+    }
+  });
+  if (tid == 0 && s_sing && status) atomicOr(&status[b], (int)ST_SINGULAR);
+}
+
+// ---------------------------------------------------------------------------
+// LU inverse of blocks up to 128 on the matrix cores, one workgroup per block
+// ---------------------------------------------------------------------------
+// The reference's algorithm: ZGETRF (partial pivoting; the pivot is the first
+// largest |Re| + |Im| of the column in the current row order, as IZAMAX picks
+// it) followed by ZGETRS against the identity (inversions.F90:807-839).
+//
+// NP = ceil(n / 16) waves; wave w holds columns 16w .. 16w+15 of all
+// R = 16 NP rows in the accumulator layout of v_mfma_f64_4x4x4: lane
+// 16a + 4b + c, strip s, quad q <-> row 16s + 4b + a, column 16w + 4q + c.
+// Rows are never moved during the elimination: pos is a row's position in
+// LAPACK's row order and a pivot step exchanges two positions.  One register
+// block holds both factors in place: a row pivoted at step k keeps U at
+// columns >= k and Y = L^-1 P left of it (unit diagonal implied), rows not
+// pivoted yet hold A right of the current step and Y left of it.
+//
+// Per panel P of 16 columns: wave P turns its columns into one row per lane
+// (two above n = 64) through its LDS scratch and runs the 16 steps alone --
+// pivot search by DPP, the pivot row by readlane, no barrier -- and publishes
+// the panel.  The other waves then add Z * (pivot rows of their own columns),
+// Z the panel's Y (L11^-1 - I on the pivot rows, -L21 L11^-1 below, 0 on rows
+// pivoted before): 64 NP instructions per wave.  A wave updates only its own
+// columns, so wave P + 1 starts its panel while the others still update.
+//
+// Then every wave sorts its rows by position and the back substitution
+// U X = Y runs by blocks of 16: U_ii X_i = Y_i row by row (explicit U_ii^-1 lost
+// a digit on nearly singular ribbon blocks), then Y_s -= U_si X_i (s < i) on the
+// matrix cores.  Operand B of these
+// products is the register block itself: block b of the instruction takes its
+// k index from quad (b + r) % 4, r = 0 .. 3, which is a DPP row rotation, and
+// A is read from LDS in the matching order.  Column j of X is column perm(j)
+// of the inverse (the row pivoted at step j).
+//
+// Bound by the panel's serial chain, instruction issue of one wave: 25 000
+// cycles per panel of 16 steps (41 000 with two rows per lane) against 7 400 per
+// update of one wave's columns (4 096 of matrix instructions at order 64).  FP32
+// blocks are converted on load and store and run in FP64.
+
+// crecip_fast without a branch (0 for b == 0), so that it overlaps the search
+__device__ inline double2 crecip_sel(double2 b) {
+  const double mx = fmax(fabs(b.x), fabs(b.y));
+  const int e = __builtin_amdgcn_frexp_exp(mx);
+  const double x = __builtin_amdgcn_ldexp(b.x, -e), y = __builtin_amdgcn_ldexp(b.y, -e);
+  const double d = fma(x, x, y * y);
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(r, fma(-d, r, 1.0), r);
+  r = fma(r, fma(-d, r, 1.0), r);
+  r = mx == 0.0 ? 0.0 : r;
+  return double2{__builtin_amdgcn_ldexp(x * r, -e), __builtin_amdgcn_ldexp(-y * r, -e)};
+}
+// f64 maximum over the wave, in every lane's SGPR copy
+template <int CTRL, int ROWS> __device__ inline double dpp_max(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  // every lane of a row pattern has a source; the broadcasts leave masked rows
+  const int l2 = ROWS == 0xF ? __builtin_amdgcn_update_dpp(0, lo, CTRL, ROWS, 0xF, true)
+                             : __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xF, false);
+  const int h2 = ROWS == 0xF ? __builtin_amdgcn_update_dpp(0, hi, CTRL, ROWS, 0xF, true)
+                             : __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xF, false);
+  return fmax(v, __hiloint2double(h2, l2));
+}
+__device__ inline double wave_fmax(double v) {
+  v = dpp_max<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v = dpp_max<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v = dpp_max<0x141, 0xF>(v);  // row_half_mirror
+  v = dpp_max<0x140, 0xF>(v);  // row_mirror
+  v = dpp_max<0x142, 0xA>(v);  // row_bcast:15
+  v = dpp_max<0x143, 0xC>(v);  // row_bcast:31
+  return lane_read(v, 63);
+}
+template <int CTRL> __device__ inline double dpp_mov(double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
+      __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
+}
+// quad (b + r) % 4 of every row of 16 lanes, into quad b
+template <int r> __device__ inline double quad_rot(double v) {
+  if constexpr (r == 0) return v;
+  else if constexpr (r == 1) return dpp_mov<0x12C>(v);  // row_ror:12
+  else if constexpr (r == 2) return dpp_mov<0x128>(v);  // row_ror:8
+  else return dpp_mov<0x124>(v);                        // row_ror:4
+}
+
+// LDS of k_lu_inv_mx<NP>, in double2: the published panel (16 columns of R + 1
+// rows) and per wave a scratch of 4 columns x R rows or of 16 x 17 pivot-row
+// entries; then the packed triangles U_ii and every U_si, s < i
+template <int NP> struct LuLds {
+  static constexpr int R = 16 * NP, LD = R + 1;
+  static constexpr int UI = 136;                 // packed 16 x 16 triangle
+  static constexpr int SHARED = 16 * LD;
+  static constexpr int SCR = 4 * R > 16 * 17 ? 4 * R : 16 * 17;
+  static constexpr int ELIM = SHARED + NP * SCR;
+  static constexpr int BACK = NP * UI + (NP * (NP - 1)) / 2 * 272;
+  static constexpr size_t bytes = (size_t)(ELIM > BACK ? ELIM : BACK) * sizeof(double2);
+};
+
+// c[q] += a b[q] for four column quads on the matrix cores; the two products of
+// an accumulator are eight instructions apart
+__device__ __forceinline__ void mfma_c4(double ar, double ai, const double (&br)[4],
+                                        const double (&bi)[4], double (&cr)[4], double (&ci)[4]) {
+  const double nai = -ai;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, br[q], cr[q], 0, 0, 0);
+    ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, bi[q], ci[q], 0, 0, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(nai, bi[q], cr[q], 0, 0, 0);
+    ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ai, br[q], ci[q], 0, 0, 0);
+  }
+}
+
+// Keeps a value's computation here: the compiler otherwise sinks the updates
+// of an unrolled section to their last use and holds all of its operands.
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void pin(double2 &v) {
+  pin(v.x);
+  pin(v.y);
+}
+// orders the LDS accesses of one wave among its own lanes
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int NP, typename IO>
+__global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_inv_mx(int n, const IO *__restrict__ A,
+                                                       long long sA, IO *__restrict__ Ainv,
+                                                       long long sAinv,
+                                                       const int *__restrict__ active,
+                                                       int *__restrict__ status) {
+  typedef double2 C;
+  typedef LuLds<NP> L;
+  constexpr int R = L::R, LD = L::LD, RT = (R + 63) / 64;
+  const int b = blockIdx.x;
+  if (active && active[b] == 0) return;
+  extern __shared__ __align__(16) unsigned char lsm[];
+  C *pan = (C *)lsm;
+  __shared__ int s_pos[R];     // position of each row
+  __shared__ int s_rowt[R];    // this panel: -1 pivoted before, 0..15 pivot step, 16 not pivoted
+  __shared__ int s_perm[R];    // row pivoted at each step
+  __shared__ C s_uinv[R];      // reciprocal pivots by step
+  __shared__ int s_sing;
+  const int tid = threadIdx.x;
+  // Wave -> columns, rotated by the dispatch round: the waves of a workgroup go
+  // to the SIMDs in order, so without it the panel waves of all workgroups that
+  // share a CU (started together) would run on one SIMD at a time.
+  const int w = __builtin_amdgcn_readfirstlane((int)((tid >> 6) + (blockIdx.x >> 8)) % NP);
+  C *scr = pan + L::SHARED + w * L::SCR;
+  int l = tid & 63;
+  int la = l >> 4, lb = (l >> 2) & 3, lc = l & 3;
+  int drow = 4 * lb + la;  // row of the lane inside a strip
+  // the lane's indices anew: addresses are then formed where they are used
+  // instead of being kept in registers across the whole kernel
+  auto fresh_lane = [&] {
+    asm volatile("" : "+v"(l));
+    la = l >> 4;
+    lb = (l >> 2) & 3;
+    lc = l & 3;
+    drow = 4 * lb + la;
+  };
+
+  // ---- load ----
+  double mr[NP][4], mi[NP][4];
+  {
+    const IO *Ab = A + (long long)b * sA;
+    static_for<NP>([&](auto S) {
+      static_for<4>([&](auto Q) {
+        const int r = 16 * S + drow, c = 16 * w + 4 * Q + lc;
+        const bool in = r < n && c < n;
+        const IO v = Ab[in ? r + c * n : 0];
+        mr[S][Q] = in ? v.x : 0.0;
+        mi[S][Q] = in ? v.y : 0.0;
+      });
+    });
+  }
+  for (int r = tid; r < R; r += 64 * NP) {
+    s_pos[r] = r;
+    s_uinv[r] = C{0, 0};
+  }
+  if (tid == 0) s_sing = 0;
+  __syncthreads();
+
+  // ---- elimination ----
+#pragma unroll 1
+  for (int P = 0; P < NP; ++P) {
+    const int kmax = min(16, n - 16 * P);
+    fresh_lane();
+    if (w == P) {
+      C v[RT][16];
+      int pos[RT], rowt[RT];
+      // own columns: one row per lane (and l + 64)
+      static_for<4>([&](auto Q) {
+        static_for<NP>([&](auto S) { scr[lc * R + 16 * S + drow] = C{mr[S][Q], mi[S][Q]}; });
+        wave_lds_fence();
+        static_for<RT>([&](auto T) {
+          const int r = min(l + 64 * T, R - 1);
+          static_for<4>([&](auto J) { v[T][4 * Q + J] = scr[J * R + r]; });
+        });
+        wave_lds_fence();
+      });
+      static_for<RT>([&](auto T) {
+        const int r = l + 64 * T;
+        pos[T] = r < n ? s_pos[r] : -1;  // padding rows count as pivoted
+        rowt[T] = pos[T] < 16 * P ? -1 : 16;
+      });
+      // Step j works on register column 0 and writes every updated column one
+      // register lower (column 0, finished, to the last), so that one loop body
+      // serves the 16 steps: unrolled, they outgrow the instruction cache.
+      // search: the lane's largest candidate in register column 0, its position
+      // and reciprocal, and the wave's maximum
+      double best, vmax;
+      int bp;
+      C rc;
+      auto search = [&](int k) {
+        best = -1.0;
+        bp = 0x7fffffff;
+        C cand = C{0, 0};
+        static_for<RT>([&](auto T) {
+          const double m = pos[T] >= k ? fabs(v[T][0].x) + fabs(v[T][0].y) : -1.0;
+          const bool hit = m > best || (T > 0 && m == best && m >= 0.0 && pos[T] < bp);
+          best = hit ? m : best;
+          bp = hit ? pos[T] : bp;
+          cand.x = hit ? v[T][0].x : cand.x;
+          cand.y = hit ? v[T][0].y : cand.y;
+        });
+        rc = crecip_sel(cand);
+        vmax = wave_fmax(best);
+      };
+      int my_p = 0;
+      C my_inv = C{0, 0};
+      bool sing = false;
+      search(16 * P);
+#pragma unroll 1
+      for (int j = 0; j < kmax; ++j) {
+        const int k = 16 * P + j;
+        unsigned long long hits = __ballot(best == vmax && bp != 0x7fffffff);
+        if (hits & (hits - 1)) {  // ties go to the smallest position
+          const unsigned key = ((hits >> l) & 1) ? (unsigned)bp : 0xFFFFFFFFu;
+          const unsigned mn = wave_min32(key);
+          hits = __ballot(key == mn);
+        }
+        if (hits == 0) {  // a column of NaN: any row left
+          bool left = false;
+          static_for<RT>([&](auto T) { left = left || pos[T] >= k; });
+          hits = __ballot(left);
+        }
+        const int pl = hits ? __ffsll((long long)hits) - 1 : 0;
+        // which of the lane's rows, and its position
+        int psel = 0;
+        if constexpr (RT > 1) psel = (pos[1] >= k && (bp == pos[1] || !(pos[0] >= k))) ? 1 : 0;
+        psel = __builtin_amdgcn_readlane(psel, pl);
+        int pp = pos[0];
+        if constexpr (RT > 1) pp = psel ? pos[1] : pos[0];
+        pp = __builtin_amdgcn_readlane(pp, pl);
+        const C pinv = C{lane_read(rc.x, pl), lane_read(rc.y, pl)};
+        // lane j keeps step j's pivot row and reciprocal
+        const bool mine = l == j;
+        my_p = mine ? pl + 64 * psel : my_p;
+        my_inv.x = mine ? pinv.x : my_inv.x;
+        my_inv.y = mine ? pinv.y : my_inv.y;
+        sing |= vmax == 0.0;
+        C m[RT], fin[RT];
+        static_for<RT>([&](auto T) {
+          const bool piv = l == pl && psel == T;
+          if (piv) {
+            pos[T] = k;
+            rowt[T] = j;
+          } else if (pos[T] == k) {
+            pos[T] = pp;
+          }
+          const bool live = pos[T] > k;
+          const C t = cmul(v[T][0], pinv);
+          m[T] = live ? t : C{0, 0};
+          // the column becomes Y's: -m below, U above and on the pivot row
+          fin[T].x = live ? -t.x : v[T][0].x;
+          fin[T].y = live ? -t.y : v[T][0].y;
+        });
+        // columns c0 .. c1-1, from the pivot row in lane pl
+        auto update = [&](auto C0, auto C1) {
+          constexpr int c0 = C0, c1 = C1;
+          C y[c1 - c0];
+          if (RT > 1 && psel)
+            static_for<c1 - c0>([&](auto I) {
+              y[I] = C{lane_read(v[RT - 1][c0 + I].x, pl), lane_read(v[RT - 1][c0 + I].y, pl)};
+            });
+          else
+            static_for<c1 - c0>([&](auto I) {
+              y[I] = C{lane_read(v[0][c0 + I].x, pl), lane_read(v[0][c0 + I].y, pl)};
+            });
+          static_for<c1 - c0>([&](auto I) {
+            static_for<RT>([&](auto T) { v[T][c0 + I - 1] = fms_c(v[T][c0 + I], m[T], y[I]); });
+          });
+        };
+        // the next column first: its search overlaps the other updates
+        update(std::integral_constant<int, 1>{}, std::integral_constant<int, 6>{});
+        search(k + 1);
+        update(std::integral_constant<int, 6>{}, std::integral_constant<int, 11>{});
+        update(std::integral_constant<int, 11>{}, std::integral_constant<int, 16>{});
+        static_for<RT>([&](auto T) { v[T][15] = fin[T]; });
+      }
+      if (l < kmax) {
+        s_perm[16 * P + l] = my_p;
+        s_uinv[16 * P + l] = my_inv;
+      }
+      if (sing && l == 0) s_sing = 1;
+      for (int j = kmax; j < 16; ++j)  // the register order after a narrow panel
+        static_for<RT>([&](auto T) {
+          const C first = v[T][0];
+          static_for<15>([&](auto Cc) { v[T][Cc] = v[T][Cc + 1]; });
+          v[T][15] = first;
+        });
+      static_for<RT>([&](auto T) {
+        const int r = l + 64 * T;
+        if (r < n) s_pos[r] = pos[T];
+      });
+      if (P > 0) __syncthreads();  // the previous panel has been read
+      static_for<RT>([&](auto T) {
+        const int r = l + 64 * T;
+        if (r < R) {
+          s_rowt[r] = rowt[T];
+          static_for<16>([&](auto Cc) { pan[Cc * LD + r] = v[T][Cc]; });
+        }
+      });
+      __syncthreads();
+      static_for<NP>([&](auto S) {
+        static_for<4>([&](auto Q) {
+          const C x = pan[(4 * Q + lc) * LD + 16 * S + drow];
+          mr[S][Q] = x.x;
+          mi[S][Q] = x.y;
+        });
+      });
+    } else {
+      if (P > 0) __syncthreads();
+      __syncthreads();
+      // pivot rows of the wave's own columns -> scratch, row t = pivot step
+      if (kmax < 16) {
+        for (int e = l; e < 16 * 17; e += 64) scr[e] = C{0, 0};
+        wave_lds_fence();
+      }
+      static_for<NP>([&](auto S) {
+        const int t = s_rowt[16 * S + drow];
+        if (t >= 0 && t < 16)
+          static_for<4>([&](auto Q) { scr[t * 17 + 4 * Q + lc] = C{mr[S][Q], mi[S][Q]}; });
+      });
+      int rt[NP];
+      static_for<NP>([&](auto S) { rt[S] = s_rowt[16 * S + (l & 15)]; });
+      wave_lds_fence();
+#pragma unroll 1
+      for (int kk = 0; kk < 4; ++kk) {
+        const int k = 4 * kk + la;
+        double br[4], bi[4];
+        static_for<4>([&](auto Q) {
+          const C x = scr[k * 17 + 4 * Q + lc];
+          br[Q] = x.x;
+          bi[Q] = x.y;
+        });
+        static_for<NP>([&](auto S) {
+          C z = pan[k * LD + 16 * S + (l & 15)];
+          if (k >= rt[S]) z = C{0, 0};
+          mfma_c4(z.x, z.y, br, bi, mr[S], mi[S]);
+        });
+      }
+      wave_lds_fence();
+    }
+  }
+
+  // ---- rows into position order ----
+  fresh_lane();
+  {
+    int ps[NP];
+    static_for<NP>([&](auto S) { ps[S] = s_pos[16 * S + drow]; });
+    static_for<4>([&](auto Q) {
+      static_for<NP>([&](auto S) { scr[lc * R + ps[S]] = C{mr[S][Q], mi[S][Q]}; });
+      wave_lds_fence();
+      static_for<NP>([&](auto S) {
+        const C x = scr[lc * R + 16 * S + drow];
+        mr[S][Q] = x.x;
+        mi[S][Q] = x.y;
+      });
+      wave_lds_fence();
+    });
+  }
+  __syncthreads();  // the last panel has been read: pan is reused
+  fresh_lane();
+  // ---- U to LDS: the triangles U_ww (packed by columns) and U_sw (s < w); the
+  // registers keep Y, unit lower triangular ----
+  C *ut = pan, *ub = pan + NP * L::UI;
+  static_for<NP>([&](auto S) {
+    if (S < w) {
+      C *u = ub + ((w * (w - 1)) / 2 + S) * 272;
+      static_for<4>([&](auto Q) {
+        u[(4 * Q + lc) * 17 + drow] = C{mr[S][Q], mi[S][Q]};
+        mr[S][Q] = 0.0;
+        mi[S][Q] = 0.0;
+      });
+    } else if (S == w) {
+      static_for<4>([&](auto Q) {
+        const int c = 4 * Q + lc;
+        if (drow <= c) ut[w * L::UI + (c * (c + 1)) / 2 + drow] = C{mr[S][Q], mi[S][Q]};
+        mr[S][Q] = c < drow ? mr[S][Q] : (c == drow ? 1.0 : 0.0);
+        mi[S][Q] = c < drow ? mi[S][Q] : 0.0;
+      });
+    }
+  });
+  __syncthreads();
+  // ---- back substitution by blocks of 16 positions, every wave on its own ----
+  static_for<NP>([&](auto K) {
+    constexpr int i = NP - 1 - K;
+    fresh_lane();
+    // U_ii X_i = Y_i row by row: row k of every column from the lanes holding it
+#pragma unroll 1
+    for (int k = 15; k >= 0; --k) {
+      const int src = (16 * (k & 3) + 4 * (k >> 2) + lc) << 2;
+      const C ui = s_uinv[16 * i + k];
+      C t = C{0, 0};
+      if (drow < k) t = ut[i * L::UI + (k * (k + 1)) / 2 + drow];
+      static_for<4>([&](auto Q) {
+        const C x = cmul(C{bperm(mr[i][Q], src), bperm(mi[i][Q], src)}, ui);
+        const C y = fms_c(C{mr[i][Q], mi[i][Q]}, t, x);
+        mr[i][Q] = drow == k ? x.x : y.x;
+        mi[i][Q] = drow == k ? x.y : y.y;
+      });
+    }
+    if constexpr (i > 0) {
+      static_for<4>([&](auto Rr) {
+        double br[4], bi[4];
+        static_for<4>([&](auto Q) {
+          br[Q] = quad_rot<Rr>(mr[i][Q]);
+          bi[Q] = quad_rot<Rr>(mi[i][Q]);
+        });
+        const int row = 4 * lb + lc, col = 4 * ((lb + Rr) & 3) + la;
+        static_for<i>([&](auto S) {
+          const C u = ub[((i * (i - 1)) / 2 + S) * 272 + col * 17 + row];
+          mfma_c4(-u.x, -u.y, br, bi, mr[S], mi[S]);
+        });
+        static_for<i>([&](auto S) {
+          static_for<4>([&](auto Q) { pin(mr[S][Q]); pin(mi[S][Q]); });
+        });
+      });
+    }
+  });
+  // ---- column j of X = U^-1 L^-1 is column perm(j) of the inverse ----
+  fresh_lane();
+  IO *Ob = Ainv + (long long)b * sAinv;
+  static_for<4>([&](auto Q) {
+    const int c = 16 * w + 4 * Q + lc;
+    if (c < n) {
+      const size_t pc = (size_t)s_perm[c] * n;
+      static_for<NP>([&](auto S) {
+        const int r = 16 * S + drow;
+        if (r < n) {
+          IO o;
+          o.x = mr[S][Q];
+          o.y = mi[S][Q];
+          Ob[r + pc] = o;
+        }
       });
     }
   });
@@ -836,30 +1208,47 @@ __global__ __launch_bounds__(NT) void k_inv_unperm(int n, const typename CT_<R>:
   }
 }
 
-template <typename R>
-size_t lds_bytes_small(int n) {
-  typedef typename CT_<R>::t C;
-  return (size_t)n * n * sizeof(C) + 2 * (size_t)n * sizeof(C) + (size_t)n * sizeof(int);
-}
-
-// largest n for the one-workgroup LDS kernel (FP32): what fits
-template <typename R>
-int lds_max_n() {
-  int n = 1;
-  while (n + 1 <= NT && lds_bytes_small<R>(n + 1) <= (size_t)kLdsBudget) ++n;
-  return n;
-}
-// largest FP64 order of the register LU kernel: 16 x 16 threads with 6 x 6
-// blocks (250 VGPRs, the U array 73 KiB at n = 96, two workgroups per CU).
-// Above it the blocked path; 2000 items of order 65 / 80 / 96 take 1.0 / 1.2 /
-// 1.7 ms here against 1.7 / 2.2 / 2.6 ms on the LDS or blocked kernels.
-constexpr int kLuMaxN = 96;
+// Largest order of the one-workgroup LU kernel, above it the blocked
+// Gauss-Jordan path.  1 / 500 / 2000 FP64 blocks, here against the thread-grid
+// LU kernel used before (us, launch and wait included): order 32 50 / 68 / 113
+// against 80 / 88 / 118, order 64 98 / 133 / 371 against 153 / 212 / 620, order
+// 96 214 / 439 / 1666 against 330 / 494 / 1702.  FP64 at order 128 the blocked
+// path is as fast (500: 0.70 against 0.84 ms, 5: 0.32 against 0.29) with smaller
+// residuals.  FP32 (the block computed in FP64): 200 blocks of order 128 take
+// 0.35 ms against 1.4 ms for Gauss-Jordan in LDS.
+template <typename R> constexpr int kLuMaxN = sizeof(R) == 8 ? 96 : 128;
 
 template <typename Kern>
 void allow_lds(Kern k, size_t bytes) {
   if (bytes > 64 * 1024)
     HN_CHECK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)bytes));
+}
+
+template <int NP, typename IO>
+void launch_lu(int n, IO *A, long long sA, IO *Ainv, long long sAinv, int batch, const int *active,
+               int *status, hipStream_t s) {
+  allow_lds(k_lu_inv_mx<NP, IO>, LuLds<NP>::bytes);
+  hipLaunchKernelGGL((k_lu_inv_mx<NP, IO>), dim3(batch), dim3(64 * NP), LuLds<NP>::bytes, s, n, A, sA,
+                     Ainv, sAinv, active, status);
+  HN_CHECK(hipGetLastError());
+}
+template <typename IO>
+void lu_mx(int n, IO *A, long long sA, IO *Ainv, long long sAinv, int batch, const int *active,
+           int *status, hipStream_t s) {
+  switch ((n + 15) / 16) {
+    case 1: return launch_lu<1>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    case 2: return launch_lu<2>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    case 3: return launch_lu<3>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    case 4: return launch_lu<4>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    case 5: return launch_lu<5>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    case 6: return launch_lu<6>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    default: break;
+  }
+  if constexpr (sizeof(IO) == sizeof(float2)) {
+    if (n <= 112) return launch_lu<7>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+    return launch_lu<8>(n, A, sA, Ainv, sAinv, batch, active, status, s);
+  }
 }
 
 template <typename R>
@@ -872,40 +1261,18 @@ void inv_impl(int n, typename CT_<R>::t *A, long long sA, typename CT_<R>::t *Ai
   const double items = w.prof_items >= 0 ? (double)w.prof_items : (active ? -1.0 : (double)batch);
   const double sm_fl = items < 0 ? -1.0 : 8.0 * (double)n * n * n * items;
   const double sm_by = items < 0 ? 0.0 : 2.0 * sizeof(typename CT_<R>::t) * (double)n * n * items;
-  if constexpr (sizeof(R) == 8) {
-    if (n <= kLuMaxN) {
-      ProfScope ps(PT_INV_SMALL, sm_fl, sm_by, s);
-      // the triangular U array: n (n - 1) / 2 entries
-      const size_t lds = std::max<size_t>(1, (size_t)n * (n - 1) / 2) * sizeof(double2);
-      if (n <= 16)
-        hipLaunchKernelGGL((k_lu_inv_2d<8, 2>), dim3(batch), dim3(64), lds, s, n, A, sA, Ainv,
-                           sAinv, active, status);
-      else if (n <= 32)
-        hipLaunchKernelGGL((k_lu_inv_2d<8, 4>), dim3(batch), dim3(64), lds, s, n, A, sA, Ainv,
-                           sAinv, active, status);
-      else if (n <= 64)
-        hipLaunchKernelGGL((k_lu_inv_2d<16, 4>), dim3(batch), dim3(256), lds, s, n, A, sA, Ainv,
-                           sAinv, active, status);
-      else if (n <= 80) {
-        allow_lds(k_lu_inv_2d<16, 5>, lds);
-        hipLaunchKernelGGL((k_lu_inv_2d<16, 5>), dim3(batch), dim3(256), lds, s, n, A, sA, Ainv,
-                           sAinv, active, status);
-      } else {
-        allow_lds(k_lu_inv_2d<16, 6>, lds);
-        hipLaunchKernelGGL((k_lu_inv_2d<16, 6>), dim3(batch), dim3(256), lds, s, n, A, sA, Ainv,
-                           sAinv, active, status);
-      }
-      HN_CHECK(hipGetLastError());
-      return;
-    }
-  }
-  if (sizeof(R) == 4 && n <= lds_max_n<R>()) {  // FP32; FP64 above kLuMaxN is blocked
-    size_t lds = lds_bytes_small<R>(n);
-    allow_lds(k_inv_lds<R>, lds);
+  if (n <= kLuMaxN<R>) {
     ProfScope ps(PT_INV_SMALL, sm_fl, sm_by, s);
-    hipLaunchKernelGGL(k_inv_lds<R>, dim3(batch), dim3(NT), lds, s, n, A, sA, Ainv, sAinv,
-                       active, status);
-    HN_CHECK(hipGetLastError());
+    if constexpr (sizeof(R) == 8) {
+      if (n <= 16) {  // one wave either way: 2000 blocks of order 10 take 32 us here, 37 below
+        const size_t lds = std::max<size_t>(1, (size_t)n * (n - 1) / 2) * sizeof(double2);
+        hipLaunchKernelGGL((k_lu_inv_2d<8, 2>), dim3(batch), dim3(64), lds, s, n, A, sA, Ainv, sAinv,
+                           active, status);
+        HN_CHECK(hipGetLastError());
+        return;
+      }
+    }
+    lu_mx(n, A, sA, Ainv, sAinv, batch, active, status, s);
     return;
   }
   if (n > 1024) throw std::runtime_error("inverse: block order > 1024 is not supported");
@@ -960,7 +1327,7 @@ void inv_impl(int n, typename CT_<R>::t *A, long long sA, typename CT_<R>::t *Ai
 
 }  // namespace
 
-int inv_lds_max_n(int real_bytes) { return real_bytes == 8 ? kLuMaxN : lds_max_n<float>(); }
+int inv_lds_max_n(int real_bytes) { return real_bytes == 8 ? kLuMaxN<double> : kLuMaxN<float>; }
 
 size_t inv_work_bytes(int n, int batch, int real_bytes) {
   size_t c = 2 * (size_t)real_bytes;

@@ -195,3 +195,44 @@ def test_gemm_tile_variants_bitwise(gpu, m, n, k, beta, ops):
     assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
     st = hip.gemm_tune_stats()
     assert st["on"] and st["shapes"] >= 1
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 48, 49, 64, 65, 79, 96, 113, 127, 128])
+def test_lu_inverse_many_blocks(gpu, n):
+    """The one-workgroup LU inverse over more blocks than one dispatch round
+    (the wave -> column rotation takes every value), with a singular block, a
+    block of equal magnitudes (pivot ties) and a NaN block among them: flags,
+    and residuals of the others at the backward error of LU with partial
+    pivoting, ||A X - I|| <= c n eps ||A|| ||X|| (c = 10 for growth)."""
+    torch, hip, eng = gpu
+    batch = 600
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn(batch, n, n, dtype=torch.complex128, device="cuda", generator=g)
+    A = A + A.mH + (0.2 + 1e-3j) * torch.eye(n, device="cuda")
+    A[7, :, n // 2] = 0.0                                # a zero column: singular
+    tie = torch.where(torch.rand(n, n, device="cuda", generator=g) < 0.5, 1.0, -1.0)
+    A[11] = tie + n * 1j * torch.eye(n, device="cuda")   # |Re| + |Im| ties off the diagonal
+    A[13, 0, n - 1] = complex(float("nan"), float("nan"))
+    X = torch.zeros_like(A)
+    st = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    W = A.clone()
+    hip.check(hip.load().hipnegf_zinverse_batched(eng.handle, n, W.data_ptr(), n * n, X.data_ptr(), n * n,
+                                                  batch, st.data_ptr()))
+    s = st.cpu().numpy()
+    assert s[7] == 1 and (np.delete(s, [7, 13]) == 0).all()
+    assert not torch.isfinite(X[13].abs()).all()
+    ok = [b for b in range(batch) if b not in (7, 13)]
+    a, x = A[ok].cpu().numpy(), X[ok].cpu().numpy()
+    res = np.linalg.norm(a @ x - np.eye(n), axis=(1, 2))
+    bound = 10 * n * 2.2e-16 * np.linalg.norm(a, axis=(1, 2)) * np.linalg.norm(x, axis=(1, 2))
+    assert (res <= bound).all(), (res / bound).max()
+    # complex FP32 in and out: the FP64 inverse of the rounded block, rounded once
+    Wc = A.to(torch.complex64)
+    Xc = torch.zeros_like(Wc)
+    hip.check(hip.load().hipnegf_cinverse_batched(eng.handle, n, Wc.data_ptr(), n * n, Xc.data_ptr(), n * n,
+                                                  batch, st.data_ptr()))
+    ac, xc = A.to(torch.complex64)[ok].cpu().numpy().astype(np.complex128), Xc[ok].cpu().numpy()
+    ref = np.linalg.inv(ac)
+    cond = np.linalg.norm(ac, axis=(1, 2)) * np.linalg.norm(ref, axis=(1, 2))
+    err = np.abs(xc - ref).max(axis=(1, 2)) / np.abs(ref).max(axis=(1, 2))
+    assert (err <= 1.2e-7 + 10 * n * 2.2e-16 * cond).all()
