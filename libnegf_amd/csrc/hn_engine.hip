@@ -2059,8 +2059,14 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
   // dephasing self-energy is diagonal; an inelastic one is fixed per call)
   double2 *Uc = arena_.take<double2>(SB * std::max(nbl - 1, 1));
   double2 *Lc = arena_.take<double2>(SB * std::max(nbl - 1, 1));
+  // products of a pass that several of its steps read, kept per interface i:
+  // ESH(i,i+1) g(i+1) from the gsmr step (Gr, Sigma_n fold), g(i+1) ESH(i+1,i)
+  // from the Gr step and g(i+1) Sigma_n(i+1) (Gn): 13 block products per
+  // interface and pass instead of 17
+  double2 *Ug = arena_.take<double2>(SB * std::max(nbl - 1, 1));
+  double2 *gL = arena_.take<double2>(SB * std::max(nbl - 1, 1));
   double2 *W1 = arena_.take<double2>(SB), *W2 = arena_.take<double2>(SB);
-  double2 *gns = arena_.take<double2>(SB), *Gnl = arena_.take<double2>(SB), *Gnu = arena_.take<double2>(SB);
+  double2 *gSn = arena_.take<double2>(SB), *Gnl = arena_.take<double2>(SB), *Gnu = arena_.take<double2>(SB);
   double2 *sig_r = arena_.take<double2>((size_t)ndev * B), *sig_n = arena_.take<double2>((size_t)ndev * B);
   double *c2 = arena_.take<double>(ndev);
   int *act = arena_.take<int>(B), *dcount = arena_.take<int>(4);
@@ -2130,29 +2136,26 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
       form_diag(nbl - 1, D);
       inverse(n, D, s2, blk(g, nbl - 1), s2, B, act, dstatus, PREC_FP64, o, n_active);
       for (int i = nbl - 2; i >= 1; --i) {
-        const double2 *U = blk(Uc, i), *L = blk(Lc, i);
         form_diag(i, D);
-        mm(U, OP_N, blk(g, i + 1), OP_N, W1, mone, zero);
-        mm(W1, OP_N, L, OP_N, D, one, one);
+        mm(blk(Uc, i), OP_N, blk(g, i + 1), OP_N, blk(Ug, i), one, zero);
+        mm(blk(Ug, i), OP_N, blk(Lc, i), OP_N, D, mone, one);
         inverse(n, D, s2, blk(g, i), s2, B, act, dstatus, PREC_FP64, o, n_active);
       }
     }
     // ---- Gr(1,1) ----
     form_diag(0, D);
     if (nbl > 1) {
-      mm(Uc, OP_N, blk(g, 1), OP_N, W1, mone, zero);
-      mm(W1, OP_N, Lc, OP_N, D, one, one);
+      mm(Uc, OP_N, blk(g, 1), OP_N, Ug, one, zero);
+      mm(Ug, OP_N, Lc, OP_N, D, mone, one);
     }
     inverse(n, D, s2, blk(Grd, 0), s2, B, act, dstatus, PREC_FP64, o, n_active);
     // ---- Gr tridiagonal blocks, i = 2..nbl (1-based) ----
     for (int i = 1; i < nbl; ++i) {
-      const double2 *U = blk(Uc, i - 1), *L = blk(Lc, i - 1);  // ESH(i-1,i), ESH(i,i-1)
-      mm(blk(g, i), OP_N, L, OP_N, W1, one, zero);
-      mm(W1, OP_N, blk(Grd, i - 1), OP_N, blk(Grl, i - 1), mone, zero);
-      mm(U, OP_N, blk(g, i), OP_N, W2, one, zero);
-      mm(blk(Grd, i - 1), OP_N, W2, OP_N, blk(Gru, i - 1), mone, zero);
+      mm(blk(g, i), OP_N, blk(Lc, i - 1), OP_N, blk(gL, i - 1), one, zero);
+      mm(blk(gL, i - 1), OP_N, blk(Grd, i - 1), OP_N, blk(Grl, i - 1), mone, zero);
+      mm(blk(Grd, i - 1), OP_N, blk(Ug, i - 1), OP_N, blk(Gru, i - 1), mone, zero);
       copy_batched(blk(Grd, i), s2, blk(g, i), s2, s2, B, act, stream_);
-      mm(blk(Grl, i - 1), OP_N, W2, OP_N, blk(Grd, i), mone, one);
+      mm(blk(Grl, i - 1), OP_N, blk(Ug, i - 1), OP_N, blk(Grd, i), mone, one);
     }
     // ---- set_Gr: sigma_r = c^2 diag(Gr) ----
     for (int i = 0; i < nbl; ++i)
@@ -2174,26 +2177,18 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
       a.active = act; a.batch = B;
       sn_form(a, stream_);
     }
-    // ---- calculate_sigma_n: upward fold ----
-    if (nbl > 1) {
-      mm(blk(g, nbl - 1), OP_N, blk(Sn, nbl - 1), OP_N, W1, one, zero);
-      mm(W1, OP_N, blk(g, nbl - 1), OP_C, gns, one, zero);
-      for (int i = nbl - 2; i >= 0; --i) {
-        const double2 *U = blk(Uc, i);
-        mm(U, OP_N, gns, OP_N, W1, one, zero);
-        mm(W1, OP_N, U, OP_C, blk(Sn, i), one, one);
-        if (inel_off) {  // Sigma_n(i,i) -= Sigma_n(i,i+1) g^H U^H + U g Sigma_n(i+1,i)
-          const double2 *snu = ist(4, i);
-          mm(snu, OP_N, blk(g, i + 1), OP_C, W1, one, zero);
-          mm(W1, OP_N, U, OP_C, blk(Sn, i), mone, one);
-          mm(U, OP_N, blk(g, i + 1), OP_N, W1, one, zero);
-          mm(W1, OP_N, snu, OP_C, blk(Sn, i), mone, one);
-        }
-        if (i > 0) {
-          mm(blk(g, i), OP_N, blk(Sn, i), OP_N, W1, one, zero);
-          mm(W1, OP_N, blk(g, i), OP_C, gns, one, zero);
-        }
+    // ---- calculate_sigma_n: upward fold, Sigma_n(i,i) += (U g) Sigma_n(i+1,i+1) (U g)^H ----
+    for (int i = nbl - 2; i >= 0; --i) {
+      const double2 *ug = blk(Ug, i);
+      if (inel_off) {  // ... - Sigma_n(i,i+1) (U g)^H - (U g) Sigma_n(i+1,i)
+        const double2 *snu = ist(4, i);
+        copy_batched(W1, s2, snu, s2, s2, B, act, stream_);
+        mm(ug, OP_N, blk(Sn, i + 1), OP_N, W1, one, mone);
+        mm(ug, OP_N, snu, OP_C, blk(Sn, i), mone, one);
+      } else {
+        mm(ug, OP_N, blk(Sn, i + 1), OP_N, W1, one, zero);
       }
+      mm(W1, OP_N, ug, OP_C, blk(Sn, i), one, one);
     }
     // ---- Gn(1,1) = Gr(1,1) Sigma_n(1,1) Gr(1,1)^H ----
     mm(blk(Sn, 0), OP_N, blk(Grd, 0), OP_C, W1, one, zero);
@@ -2201,23 +2196,23 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
     fill_int(reinterpret_cast<int *>(err), 2 * B, 0, stream_);
     // ---- downward recursion ----
     for (int i = 0; i + 1 < nbl; ++i) {
-      const double2 *L = blk(Lc, i);  // ESH(i+1,i)
       // with inelastic stores, Gn(i+1,i) / Gn(i,i+1) are formed in them directly
       // (cache_Gn; masked launches leave converged items' blocks as they were)
       double2 *Gnl_i = io ? ost(5, i) : Gnl, *Gnu_i = io ? ost(4, i) : Gnu;
-      mm(blk(Sn, i + 1), OP_N, blk(Gru, i), OP_C, W1, one, zero);
-      if (inel_off) mm(ist(4, i), OP_C, blk(Grd, i), OP_C, W1, one, one);  // Sigma_n(i+1,i) Gr(i,i)^H
-      mm(L, OP_N, blk(Gnd, i), OP_N, W1, mone, one);
-      mm(blk(g, i + 1), OP_N, W1, OP_N, Gnl_i, one, zero);
-      // Gn(i,i+1) = Gn(i+1,i)^H is formed only where it is kept or tested;
-      // otherwise the product below reads Gn(i+1,i) conjugate-transposed
-      const bool keep_gnu = io || s_general;
-      if (keep_gnu) dagger_batched(Gnl_i, s2, Gnu_i, s2, n, n, B, act, stream_);
-      mm(blk(Sn, i + 1), OP_N, blk(Grd, i + 1), OP_C, W1, one, zero);
-      if (inel_off) mm(ist(4, i), OP_C, blk(Grl, i), OP_C, W1, one, one);  // Sigma_n(i+1,i) Gr(i+1,i)^H
-      if (keep_gnu) mm(L, OP_N, Gnu_i, OP_N, W1, mone, one);
-      else mm(L, OP_N, Gnl_i, OP_C, W1, mone, one);
-      mm(blk(g, i + 1), OP_N, W1, OP_N, blk(Gnd, i + 1), one, zero);
+      // Gn(i+1,i) = g Sn(i+1) Gr(i,i+1)^H + g Sigma_n(i+1,i) Gr(i,i)^H - g L Gn(i,i)
+      mm(blk(g, i + 1), OP_N, blk(Sn, i + 1), OP_N, gSn, one, zero);
+      mm(gSn, OP_N, blk(Gru, i), OP_C, Gnl_i, one, zero);
+      if (inel_off) {
+        mm(blk(g, i + 1), OP_N, ist(4, i), OP_C, W2, one, zero);
+        mm(W2, OP_N, blk(Grd, i), OP_C, Gnl_i, one, one);
+      }
+      mm(blk(gL, i), OP_N, blk(Gnd, i), OP_N, Gnl_i, mone, one);
+      // Gn(i,i+1) = Gn(i+1,i)^H is formed only where it is kept or tested
+      if (io || s_general) dagger_batched(Gnl_i, s2, Gnu_i, s2, n, n, B, act, stream_);
+      // Gn(i+1,i+1), the same with Gr(i+1,i+1), Gr(i+1,i) and Gn(i,i+1)
+      mm(gSn, OP_N, blk(Grd, i + 1), OP_C, blk(Gnd, i + 1), one, zero);
+      if (inel_off) mm(W2, OP_N, blk(Grl, i), OP_C, blk(Gnd, i + 1), one, one);
+      mm(blk(gL, i), OP_N, Gnl_i, OP_C, blk(Gnd, i + 1), mone, one);
       if (s_general) {  // off-diagonal S entries enter the convergence test
         // Gn(i+1,i) = Gn(i,i+1)^H, so |dGn(i+1,i)(r,c)| = |dGn(i,i+1)(c,r)|: one pass over
         // Gn(i,i+1) with the union of the S(i,i+1) pattern and the transposed S(i+1,i) pattern
@@ -2278,9 +2273,9 @@ void Engine::scba_mw(DevStruct &st, int nitems, const double *dE, const int *dsl
   // n: the (uniform) PL order; nm >= n also covers contact surface blocks
   const int n = st.bsz[0], nm = st.nmax(), nbl = st.nbl;
   const size_t b2 = (size_t)nm * nm * sizeof(double2);
-  // G^r/G^n block lists and ESH off-diagonal blocks (11 nbl) + sweep temporaries (8) + contact decimation and
+  // G^r/G^n block lists, ESH off-diagonal blocks and kept products (13 nbl) + sweep temporaries (8) + contact decimation and
   // self-energy workspace (12 per contact) + inverse workspace + per-orbital vectors
-  const size_t per_item = b2 * (size_t)(11 * nbl + 12 * st.ncont + 16) +
+  const size_t per_item = b2 * (size_t)(13 * nbl + 12 * st.ncont + 16) +
                           inv_work_bytes(nm, std::max(st.ncont, 1), 8) + (size_t)n * nbl * 48 + 1024;
   const int B = pick_batch(st, nitems, o, per_item);
   last_batch_ = B;
@@ -2431,7 +2426,7 @@ void Engine::inel_mw(DevStruct &st, const double *E, const double *frm, const So
   // batch of the elastic sweeps (same per-item budget as scba_mw)
   const int nm = st.nmax();
   const size_t b2 = (size_t)nm * nm * sizeof(double2);
-  const size_t per_item = b2 * (size_t)(11 * nbl + 12 * ncont + 16) +
+  const size_t per_item = b2 * (size_t)(13 * nbl + 12 * ncont + 16) +
                           inv_work_bytes(nm, ncont, 8) + (size_t)n * nbl * 48 + 1024;
   const int B = pick_batch(st, (int)std::min<long long>(NI, 1 << 30), o, per_item);
   last_batch_ = B;
