@@ -50,11 +50,16 @@ struct FusedLayout {
   __device__ long long cnt(int c, int k) const { return offs[2 * nbl + 4 * (nbl - 1) + 6 * c + k]; }
 };
 
-// One wave (64 lanes) per item.  Every helper is called by all 64 lanes and
-// ends with a barrier, so LDS results are visible to the next call.
+// Helpers of one wave on its own LDS blocks: each is called by all 64 lanes and
+// ends with a fence that orders the wave's LDS accesses, so results are visible
+// to the next call (the waves of a workgroup never share a block in between).
 struct Wave {
   int n, lane;
-  __device__ void sync() const { __syncthreads(); }
+  __device__ void sync() const {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 
   // out = z S - H (S absent: identity if sid, else zero); dag: its conjugate
   // transpose
@@ -181,9 +186,14 @@ struct Wave {
   }
 };
 
-constexpr int kFusedMats = 12;
+// LDS blocks of an item: ten per wave and the two self-energies.  One wave per
+// item decimates the contacts one after the other; with two (NW = 2) each wave
+// takes one contact and the first goes on with the sweep: the same operations
+// on every element, the decimations (two thirds of the chain) side by side.
+constexpr int fused_mats(int nw) { return 10 * nw + 2; }
 
-__global__ __launch_bounds__(64) void k_t_fused(FusedLayout L, int nitems, const double *E,
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_t_fused(FusedLayout L, int nitems, const double *E,
                                                 const int *slot, double delta, double sgfacc,
                                                 int crit, int maxit, double *T, int *ncyc,
                                                 int *status) {
@@ -191,17 +201,21 @@ __global__ __launch_bounds__(64) void k_t_fused(FusedLayout L, int nitems, const
   if (b >= nitems) return;
   extern __shared__ __align__(16) unsigned char fsm[];
   const int n = L.n, nn = n * n;
-  C *M[kFusedMats];
-  for (int i = 0; i < kFusedMats; ++i) M[i] = (C *)fsm + (size_t)i * nn;
-  int *piv = (int *)((C *)fsm + (size_t)kFusedMats * nn);
-  Wave w{n, (int)threadIdx.x};
+  const int wv = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  C *own = (C *)fsm + (size_t)(10 * wv) * nn;
+  C *M[10];
+  for (int i = 0; i < 10; ++i) M[i] = own + (size_t)i * nn;
+  int *piv = (int *)((C *)fsm + (size_t)fused_mats(NW) * nn) + 64 * wv;
+  __shared__ int s_st;
+  if (NW > 1 && threadIdx.x == 0) s_st = 0;
+  Wave w{n, (int)threadIdx.x & 63};
   const C *base = L.pool + (long long)slot[b] * L.slot_stride;
   auto blk = [&](long long off) -> const C * { return off < 0 ? nullptr : base + off; };
   const double er = E[b];
   int st = 0;
-  C *Sig[2] = {M[10], M[11]};
+  C *Sig[2] = {(C *)fsm + (size_t)(10 * NW) * nn, (C *)fsm + (size_t)(10 * NW + 1) * nn};
 
-  for (int c = 0; c < 2; ++c) {
+  for (int c = wv; c < 2; c += NW) {
     C *Ao = M[0], *Aos = M[1], *Bo = M[2], *Co = M[3], *Go = M[4];
     C *GC = M[5], *C1 = M[6], *GB = M[7], *B1 = M[8], *LU = M[9];
     const C *H00 = blk(L.cnt(c, 0)), *S00 = blk(L.cnt(c, 1));
@@ -256,7 +270,14 @@ __global__ __launch_bounds__(64) void k_t_fused(FusedLayout L, int nitems, const
     w.mm(Sig[c], GB, C1, 0);
     if (w.lane == 0 && ncyc) ncyc[(long long)b * 2 + c] = nc;
     // restore the buffer table for the next contact
-    for (int i = 0; i < 10; ++i) M[i] = (C *)fsm + (size_t)i * nn;
+    for (int i = 0; i < 10; ++i) M[i] = own + (size_t)i * nn;
+  }
+  if constexpr (NW > 1) {
+    __syncthreads();  // s_st is cleared
+    if (w.lane == 0 && st) atomicOr(&s_st, st);
+    __syncthreads();  // both self-energies are in place
+    if (wv != 0) return;
+    st = s_st;
   }
 
   // backward sweep at real E: g_nbl = ESH_nbl^-1, g_i = (ESH_ii - ESH_i,i+1 g ESH_i+1,i)^-1
@@ -342,11 +363,27 @@ bool Engine::t_fused(DevStruct &st, int nitems, const double *dE, const int *dsl
   L.offs = doffs;
   L.slot_stride = st.slot_elems;
   L.pool = st.pool;
-  const size_t lds = (size_t)kFusedMats * n * n * sizeof(double2) + 64 * sizeof(int);
+  auto lds_of = [&](int W) {
+    return (size_t)fused_mats(W) * n * n * sizeof(double2) + (size_t)W * 64 * sizeof(int);
+  };
+  // Two waves per item while all items are resident at once (256 CUs of 160 KiB
+  // LDS): the call then takes one item's chain (200 items of 20 layers, order 10:
+  // 1.83 -> 1.23 ms; order 16: 3.98 -> 2.57).  Beyond that the LDS per item
+  // decides, twelve blocks against twenty-two (order 16, 500 items: 4.1 ms with
+  // one wave each).
+  const long long fit2 = 256LL * (long long)((160 * 1024 - 1024) / (lds_of(2) + 256));
+  const bool two = nitems <= fit2;
   {
     ProfScope ps(PT_FUSED, -1.0, 0.0, stream_);
-    hipLaunchKernelGGL(k_t_fused, dim3(nitems), dim3(64), lds, stream_, L, nitems, dE, dslot,
-                       o.delta, o.sgfacc, o.dec_crit, o.dec_maxit, dT, dncyc, dstatus);
+    if (two) {
+      HN_CHECK(hipFuncSetAttribute((const void *)k_t_fused<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)lds_of(2)));
+      hipLaunchKernelGGL(k_t_fused<2>, dim3(nitems), dim3(128), lds_of(2), stream_, L, nitems, dE, dslot,
+                         o.delta, o.sgfacc, o.dec_crit, o.dec_maxit, dT, dncyc, dstatus);
+    } else {
+      hipLaunchKernelGGL(k_t_fused<1>, dim3(nitems), dim3(64), lds_of(1), stream_, L, nitems, dE, dslot,
+                         o.delta, o.sgfacc, o.dec_crit, o.dec_maxit, dT, dncyc, dstatus);
+    }
     HN_CHECK(hipGetLastError());
   }
   HN_CHECK(hipStreamSynchronize(stream_));  // the offset table's host copy stays valid until here
