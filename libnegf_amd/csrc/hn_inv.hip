@@ -17,6 +17,7 @@
 // accumulated transform; the other columns of M then take ONE deferred
 // rank-|S| update on the matrix cores.  After the last super-panel,
 // M^-1(i, c) = B(pi(i), pi^-1(c)) with pi(c) the pivot row of column c.
+#include <cfloat>
 #include <utility>
 
 #include "hn_gemm.h"
@@ -611,7 +612,9 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
         bp = 0x7fffffff;
         C cand = C{0, 0};
         static_for<RT>([&](auto T) {
-          const double m = pos[T] >= k ? fabs(v[T][0].x) + fabs(v[T][0].y) : -1.0;
+          // NaN and Inf count as the largest finite number: a NaN is a pivot like
+          // any other and spreads over the inverse
+          const double m = pos[T] >= k ? fmin(fabs(v[T][0].x) + fabs(v[T][0].y), DBL_MAX) : -1.0;
           const bool hit = m > best || (T > 0 && m == best && m >= 0.0 && pos[T] < bp);
           best = hit ? m : best;
           bp = hit ? pos[T] : bp;
@@ -634,20 +637,26 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
           const unsigned mn = wave_min32(key);
           hits = __ballot(key == mn);
         }
-        if (hits == 0) {  // a column of NaN: any row left
-          bool left = false;
-          static_for<RT>([&](auto T) { left = left || pos[T] >= k; });
-          hits = __ballot(left);
-        }
-        const int pl = hits ? __ffsll((long long)hits) - 1 : 0;
+        const int pl = __ffsll((long long)hits) - 1;  // n - k rows are left
         // which of the lane's rows, and its position
         int psel = 0;
-        if constexpr (RT > 1) psel = (pos[1] >= k && (bp == pos[1] || !(pos[0] >= k))) ? 1 : 0;
+        if constexpr (RT > 1) psel = bp == pos[1] ? 1 : 0;
         psel = __builtin_amdgcn_readlane(psel, pl);
         int pp = pos[0];
         if constexpr (RT > 1) pp = psel ? pos[1] : pos[0];
         pp = __builtin_amdgcn_readlane(pp, pl);
-        const C pinv = C{lane_read(rc.x, pl), lane_read(rc.y, pl)};
+        C pinv = C{lane_read(rc.x, pl), lane_read(rc.y, pl)};
+        if constexpr (sizeof(IO) == sizeof(float2))
+          if (vmax == DBL_MAX) {  // FP32: a NaN is flagged, the reciprocal of Inf is 0
+            double px = lane_read(v[0][0].x, pl), py = lane_read(v[0][0].y, pl);
+            if constexpr (RT > 1) {
+              const double qx = lane_read(v[1][0].x, pl), qy = lane_read(v[1][0].y, pl);
+              px = psel ? qx : px;
+              py = psel ? qy : py;
+            }
+            pinv = crecip(C{px, py});
+            sing |= px != px || py != py;
+          }
         // lane j keeps step j's pivot row and reciprocal
         const bool mine = l == j;
         my_p = mine ? pl + 64 * psel : my_p;

@@ -236,3 +236,40 @@ def test_lu_inverse_many_blocks(gpu, n):
     cond = np.linalg.norm(ac, axis=(1, 2)) * np.linalg.norm(ref, axis=(1, 2))
     err = np.abs(xc - ref).max(axis=(1, 2)) / np.abs(ref).max(axis=(1, 2))
     assert (err <= 1.2e-7 + 10 * n * 2.2e-16 * cond).all()
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 40, 64, 65, 96, 97, 128])
+def test_lu_inverse_nonfinite(gpu, n):
+    """Blocks holding a NaN in any corner or in the middle: nothing finite in the
+    FP64 inverse (orders up to 96), whichever row is pivoted when, and in FP32
+    the singular flag; an infinite FP32 pivot has the reciprocal 0, so its row
+    and column of the inverse vanish and the rest is the inverse of the rest."""
+    torch, hip, eng = gpu
+    g = torch.Generator(device="cuda").manual_seed(n)
+    at = [(0, 0), (0, n - 1), (n - 1, 0), (n - 1, n - 1), (n // 2, n // 3), (n // 3, n // 2)]
+    A = torch.randn(len(at) + 2, n, n, dtype=torch.complex128, device="cuda", generator=g)
+    A = A + 0.2j * torch.eye(n, device="cuda")
+    for b, (i, j) in enumerate(at):
+        A[b, i, j] = complex(float("nan"), float("nan"))
+    nan = range(len(at))
+    for typ, f in (("z", hip.load().hipnegf_zinverse_batched), ("c", hip.load().hipnegf_cinverse_batched)):
+        if typ == "z" and n > 96:
+            continue
+        W = A.clone() if typ == "z" else A.to(torch.complex64)
+        if typ == "c":
+            W[-1, 0, 0] = float("inf")
+        W0 = W.clone()
+        X = torch.zeros_like(W)
+        st = torch.zeros(len(W), dtype=torch.int32, device="cuda")
+        hip.check(f(eng.handle, n, W.data_ptr(), n * n, X.data_ptr(), n * n, len(W), st.data_ptr()))
+        s, x, w = st.cpu().numpy(), X.cpu().numpy(), W0.cpu().numpy()
+        if typ == "z":
+            assert not np.isfinite(x[nan].real).any() and not np.isfinite(x[nan].imag).any()
+            assert (s[len(at):] == 0).all()
+            continue
+        assert (s[nan] == 1).all() and (s[len(at):] == 0).all()
+        assert not np.isfinite(x[nan]).all(axis=(1, 2)).any()
+        assert (x[-1][0] == 0).all() and (x[-1][:, 0] == 0).all()
+        if n > 1:
+            r = w[-1][1:, 1:].astype(np.complex128) @ x[-1][1:, 1:] - np.eye(n - 1)
+            assert np.linalg.norm(r) <= 1e-5 * np.linalg.norm(w[-1][1:, 1:]) * np.linalg.norm(x[-1])
