@@ -408,13 +408,19 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
 // columns >= k and Y = L^-1 P left of it (unit diagonal implied), rows not
 // pivoted yet hold A right of the current step and Y left of it.
 //
-// Per panel P of 16 columns: wave P turns its columns into one row per lane
-// (two above n = 64) through its LDS scratch and runs the 16 steps alone --
+// Per panel of 4 columns: the wave that owns them turns them into one row per
+// lane (two above n = 64) through its LDS scratch and runs the 4 steps alone --
 // pivot search by DPP, the pivot row by readlane, no barrier -- and publishes
-// the panel.  The other waves then add Z * (pivot rows of their own columns),
-// Z the panel's Y (L11^-1 - I on the pivot rows, -L21 L11^-1 below, 0 on rows
-// pivoted before): 64 NP instructions per wave.  A wave updates only its own
-// columns, so wave P + 1 starts its panel while the others still update.
+// the panel (two buffers, one barrier per panel).  Every wave then adds
+// Z * (pivot rows of its own columns), Z the panel's Y (L11^-1 - I on the pivot
+// rows, -L21 L11^-1 below, 0 on rows pivoted before): one K = 4 product, 16 NP
+// matrix instructions per wave.  Four columns, since the explicit L11^-1 costs
+// accuracy as it grows: on blocks with random +-0.97 multipliers 16 columns gave
+// 2.4 - 2.9 times LAPACK's error, four give 0.95 - 0.99, and the transmission of
+// ribbons of 24 to 90 orbitals had 4 - 22 % more error in the mean over 800
+// energies than elimination one column at a time, now 4 % more to 6 % less.  And
+// since four columns take 16 registers per row of a lane, so that two workgroups
+// of 5 or 6 waves share a CU.
 //
 // Then every wave sorts its rows by position and the back substitution
 // U X = Y runs by blocks of 16: U_ii X_i = Y_i row by row (explicit U_ii^-1 lost
@@ -425,12 +431,13 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
 // A is read from LDS in the matching order.  Column j of X is column perm(j)
 // of the inverse (the row pivoted at step j).
 //
-// Bound by the panel's serial chain, instruction issue of one wave: 25 000
-// cycles per panel of 16 steps (41 000 with two rows per lane) against 7 400 per
-// update of one wave's columns (4 096 of matrix instructions at order 64).  FP32
-// blocks are converted on load and store and run in FP64.
+// FP32 blocks are converted on load and store and run in FP64.
 
-// crecip_fast without a branch (0 for b == 0), so that it overlaps the search
+// 1/b for a pivot without a branch, so that it overlaps the search (0 for
+// b == 0): b scaled as in crecip_fast, one Newton-Raphson step on 1/|b'|^2 and
+// one on the complex reciprocal itself, p <- p + p (1 - b p), which leaves
+// little but the rounding of p (inverses of a ribbon's first decimation step:
+// error 3.2e-16, with crecip_fast's two real steps 3.5e-16)
 __device__ inline double2 crecip_sel(double2 b) {
   const double mx = fmax(fabs(b.x), fabs(b.y));
   const int e = __builtin_amdgcn_frexp_exp(mx);
@@ -438,9 +445,11 @@ __device__ inline double2 crecip_sel(double2 b) {
   const double d = fma(x, x, y * y);
   double r = __builtin_amdgcn_rcp(d);
   r = fma(r, fma(-d, r, 1.0), r);
-  r = fma(r, fma(-d, r, 1.0), r);
   r = mx == 0.0 ? 0.0 : r;
-  return double2{__builtin_amdgcn_ldexp(x * r, -e), __builtin_amdgcn_ldexp(-y * r, -e)};
+  const double px = x * r, py = -y * r;
+  const double er = fma(y, py, fma(-x, px, 1.0)), ei = fma(-y, px, -x * py);
+  return double2{__builtin_amdgcn_ldexp(fma(-py, ei, fma(px, er, px)), -e),
+                 __builtin_amdgcn_ldexp(fma(px, ei, fma(py, er, py)), -e)};
 }
 // f64 maximum over the wave, in every lane's SGPR copy
 template <int CTRL, int ROWS> __device__ inline double dpp_max(double v) {
@@ -474,33 +483,42 @@ template <int r> __device__ inline double quad_rot(double v) {
   else return dpp_mov<0x124>(v);                        // row_ror:4
 }
 
-// LDS of k_lu_inv_mx<NP>, in double2: the published panel (16 columns of R + 1
-// rows) and per wave a scratch of 4 columns x R rows or of 16 x 17 pivot-row
+// LDS of k_lu_inv_mx<NP>, in double2: two published panels (4 columns of R + 1
+// rows each) and per wave a scratch of 4 columns x R rows or of 4 x 17 pivot-row
 // entries; then the packed triangles U_ii and every U_si, s < i
 template <int NP> struct LuLds {
   static constexpr int R = 16 * NP, LD = R + 1;
   static constexpr int UI = 136;                 // packed 16 x 16 triangle
-  static constexpr int SHARED = 16 * LD;
-  static constexpr int SCR = 4 * R > 16 * 17 ? 4 * R : 16 * 17;
+  static constexpr int SHARED = 2 * 4 * LD;
+  static constexpr int SCR = 4 * R > 4 * 17 ? 4 * R : 4 * 17;
   static constexpr int ELIM = SHARED + NP * SCR;
   static constexpr int BACK = NP * UI + (NP * (NP - 1)) / 2 * 272;
   static constexpr size_t bytes = (size_t)(ELIM > BACK ? ELIM : BACK) * sizeof(double2);
 };
 
-// c[q] += a b[q] for four column quads on the matrix cores; the two products of
-// an accumulator are eight instructions apart
+// c[q] += a b[q] for four column quads on the matrix cores, the K = 4 products
+// summed apart and added once: into c itself every one of their eight terms is
+// rounded at the size of c (inverses of a ribbon's converged surface blocks and
+// of its sweep blocks, order 64: error 8.0e-16 and 16e-16, apart 3.9e-16 and
+// 7.8e-16; 3 % longer)
 __device__ __forceinline__ void mfma_c4(double ar, double ai, const double (&br)[4],
                                         const double (&bi)[4], double (&cr)[4], double (&ci)[4]) {
   const double nai = -ai;
+  double tr[4], ti[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, br[q], cr[q], 0, 0, 0);
-    ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, bi[q], ci[q], 0, 0, 0);
+    tr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, br[q], 0.0, 0, 0, 0);
+    ti[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, bi[q], 0.0, 0, 0, 0);
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(nai, bi[q], cr[q], 0, 0, 0);
-    ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ai, br[q], ci[q], 0, 0, 0);
+    tr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(nai, bi[q], tr[q], 0, 0, 0);
+    ti[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(ai, br[q], ti[q], 0, 0, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    cr[q] += tr[q];
+    ci[q] += ti[q];
   }
 }
 
@@ -518,8 +536,11 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// waves per SIMD the registers are kept for: whole workgroups of NP waves
+constexpr int lu_waves(int np) { return np <= 4 ? 4 : np <= 6 ? 3 : 2; }
+
 template <int NP, typename IO>
-__global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_inv_mx(int n, const IO *__restrict__ A,
+__global__ __launch_bounds__(64 * NP, lu_waves(NP)) void k_lu_inv_mx(int n, const IO *__restrict__ A,
                                                        long long sA, IO *__restrict__ Ainv,
                                                        long long sAinv,
                                                        const int *__restrict__ active,
@@ -532,7 +553,7 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
   extern __shared__ __align__(16) unsigned char lsm[];
   C *pan = (C *)lsm;
   __shared__ int s_pos[R];     // position of each row
-  __shared__ int s_rowt[R];    // this panel: -1 pivoted before, 0..15 pivot step, 16 not pivoted
+  __shared__ int s_rowt[2][R];  // a panel's rows: -1 pivoted before, 0..3 pivot step, 4 not pivoted
   __shared__ int s_perm[R];    // row pivoted at each step
   __shared__ C s_uinv[R];      // reciprocal pivots by step
   __shared__ int s_sing;
@@ -579,193 +600,145 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
   // ---- elimination ----
 #pragma unroll 1
   for (int P = 0; P < NP; ++P) {
-    const int kmax = min(16, n - 16 * P);
-    fresh_lane();
-    if (w == P) {
-      C v[RT][16];
-      int pos[RT], rowt[RT];
-      // own columns: one row per lane (and l + 64)
-      static_for<4>([&](auto Q) {
-        static_for<NP>([&](auto S) { scr[lc * R + 16 * S + drow] = C{mr[S][Q], mi[S][Q]}; });
+    static_for<4>([&](auto G) {
+      constexpr int buf = G & 1;
+      const int k0 = 16 * P + 4 * G, kmax = min(4, n - k0);
+      if (kmax <= 0) return;  // uniform
+      C *pn = pan + buf * 4 * LD;
+      fresh_lane();
+      if (w == P) {
+        C v[RT][4];
+        int pos[RT], rowt[RT];
+        // own columns: one row per lane (and l + 64)
+        static_for<NP>([&](auto S) { scr[lc * R + 16 * S + drow] = C{mr[S][G], mi[S][G]}; });
         wave_lds_fence();
         static_for<RT>([&](auto T) {
-          const int r = min(l + 64 * T, R - 1);
-          static_for<4>([&](auto J) { v[T][4 * Q + J] = scr[J * R + r]; });
+          const int r = l + 64 * T, rr = min(r, R - 1);
+          static_for<4>([&](auto J) { v[T][J] = scr[J * R + rr]; });
+          pos[T] = r < n ? s_pos[r] : -1;  // padding rows count as pivoted
+          rowt[T] = pos[T] < k0 ? -1 : 4;
         });
-        wave_lds_fence();
-      });
-      static_for<RT>([&](auto T) {
-        const int r = l + 64 * T;
-        pos[T] = r < n ? s_pos[r] : -1;  // padding rows count as pivoted
-        rowt[T] = pos[T] < 16 * P ? -1 : 16;
-      });
-      // Step j works on register column 0 and writes every updated column one
-      // register lower (column 0, finished, to the last), so that one loop body
-      // serves the 16 steps: unrolled, they outgrow the instruction cache.
-      // search: the lane's largest candidate in register column 0, its position
-      // and reciprocal, and the wave's maximum
-      double best, vmax;
-      int bp;
-      C rc;
-      auto search = [&](int k) {
-        best = -1.0;
-        bp = 0x7fffffff;
-        C cand = C{0, 0};
-        static_for<RT>([&](auto T) {
-          // NaN and Inf count as the largest finite number: a NaN is a pivot like
-          // any other and spreads over the inverse
-          const double m = pos[T] >= k ? fmin(fabs(v[T][0].x) + fabs(v[T][0].y), DBL_MAX) : -1.0;
-          const bool hit = m > best || (T > 0 && m == best && m >= 0.0 && pos[T] < bp);
-          best = hit ? m : best;
-          bp = hit ? pos[T] : bp;
-          cand.x = hit ? v[T][0].x : cand.x;
-          cand.y = hit ? v[T][0].y : cand.y;
-        });
-        rc = crecip_sel(cand);
-        vmax = wave_fmax(best);
-      };
-      int my_p = 0;
-      C my_inv = C{0, 0};
-      bool sing = false;
-      search(16 * P);
-#pragma unroll 1
-      for (int j = 0; j < kmax; ++j) {
-        const int k = 16 * P + j;
-        unsigned long long hits = __ballot(best == vmax && bp != 0x7fffffff);
-        if (hits & (hits - 1)) {  // ties go to the smallest position
-          const unsigned key = ((hits >> l) & 1) ? (unsigned)bp : 0xFFFFFFFFu;
-          const unsigned mn = wave_min32(key);
-          hits = __ballot(key == mn);
-        }
-        const int pl = __ffsll((long long)hits) - 1;  // n - k rows are left
-        // which of the lane's rows, and its position
-        int psel = 0;
-        if constexpr (RT > 1) psel = bp == pos[1] ? 1 : 0;
-        psel = __builtin_amdgcn_readlane(psel, pl);
-        int pp = pos[0];
-        if constexpr (RT > 1) pp = psel ? pos[1] : pos[0];
-        pp = __builtin_amdgcn_readlane(pp, pl);
-        C pinv = C{lane_read(rc.x, pl), lane_read(rc.y, pl)};
-        if constexpr (sizeof(IO) == sizeof(float2))
-          if (vmax == DBL_MAX) {  // FP32: a NaN is flagged, the reciprocal of Inf is 0
-            double px = lane_read(v[0][0].x, pl), py = lane_read(v[0][0].y, pl);
-            if constexpr (RT > 1) {
-              const double qx = lane_read(v[1][0].x, pl), qy = lane_read(v[1][0].y, pl);
-              px = psel ? qx : px;
-              py = psel ? qy : py;
+        bool sing = false;
+        static_for<4>([&](auto J) {
+          constexpr int j = J;
+          const int k = k0 + j;
+          if (k >= n) return;  // uniform
+          // the lane's largest candidate, its position and reciprocal, and the
+          // wave's maximum; NaN and Inf count as the largest finite number: a
+          // NaN is a pivot like any other and spreads over the inverse
+          double best = -1.0;
+          int bp = 0x7fffffff;
+          C cand = C{0, 0};
+          static_for<RT>([&](auto T) {
+            const double m = pos[T] >= k ? fmin(fabs(v[T][j].x) + fabs(v[T][j].y), DBL_MAX) : -1.0;
+            const bool hit = m > best || (T > 0 && m == best && m >= 0.0 && pos[T] < bp);
+            best = hit ? m : best;
+            bp = hit ? pos[T] : bp;
+            cand.x = hit ? v[T][j].x : cand.x;
+            cand.y = hit ? v[T][j].y : cand.y;
+          });
+          const C rc = crecip_sel(cand);
+          const double vmax = wave_fmax(best);
+          unsigned long long hits = __ballot(best == vmax && bp != 0x7fffffff);
+          if (hits & (hits - 1)) {  // ties go to the smallest position
+            const unsigned key = ((hits >> l) & 1) ? (unsigned)bp : 0xFFFFFFFFu;
+            const unsigned mn = wave_min32(key);
+            hits = __ballot(key == mn);
+          }
+          const int pl = __ffsll((long long)hits) - 1;  // n - k rows are left
+          // which of the lane's rows, and its position
+          int psel = 0;
+          if constexpr (RT > 1) psel = __builtin_amdgcn_readlane(bp == pos[1] ? 1 : 0, pl);
+          const int pp = __builtin_amdgcn_readlane(bp, pl);
+          C pinv = C{lane_read(rc.x, pl), lane_read(rc.y, pl)};
+          if constexpr (sizeof(IO) == sizeof(float2))
+            if (vmax == DBL_MAX) {  // FP32: a NaN is flagged, the reciprocal of Inf is 0
+              const double px = lane_read(cand.x, pl), py = lane_read(cand.y, pl);
+              pinv = crecip(C{px, py});
+              sing |= px != px || py != py;
             }
-            pinv = crecip(C{px, py});
-            sing |= px != px || py != py;
+          sing |= vmax == 0.0;
+          if (l == j) {
+            s_perm[k] = pl + 64 * psel;
+            s_uinv[k] = pinv;
           }
-        // lane j keeps step j's pivot row and reciprocal
-        const bool mine = l == j;
-        my_p = mine ? pl + 64 * psel : my_p;
-        my_inv.x = mine ? pinv.x : my_inv.x;
-        my_inv.y = mine ? pinv.y : my_inv.y;
-        sing |= vmax == 0.0;
-        C m[RT], fin[RT];
-        static_for<RT>([&](auto T) {
-          const bool piv = l == pl && psel == T;
-          if (piv) {
-            pos[T] = k;
-            rowt[T] = j;
-          } else if (pos[T] == k) {
-            pos[T] = pp;
-          }
-          const bool live = pos[T] > k;
-          const C t = cmul(v[T][0], pinv);
-          m[T] = live ? t : C{0, 0};
-          // the column becomes Y's: -m below, U above and on the pivot row
-          fin[T].x = live ? -t.x : v[T][0].x;
-          fin[T].y = live ? -t.y : v[T][0].y;
-        });
-        // columns c0 .. c1-1, from the pivot row in lane pl
-        auto update = [&](auto C0, auto C1) {
-          constexpr int c0 = C0, c1 = C1;
-          C y[c1 - c0];
+          C m[RT];
+          static_for<RT>([&](auto T) {
+            const bool piv = l == pl && psel == T;
+            if (piv) {
+              pos[T] = k;
+              rowt[T] = j;
+            } else if (pos[T] == k) {
+              pos[T] = pp;
+            }
+            const bool live = pos[T] > k;
+            const C t = cmul(v[T][j], pinv);
+            m[T] = live ? t : C{0, 0};
+          });
+          // the other columns, from the pivot row in lane pl
+          C y[4];
           if (RT > 1 && psel)
-            static_for<c1 - c0>([&](auto I) {
-              y[I] = C{lane_read(v[RT - 1][c0 + I].x, pl), lane_read(v[RT - 1][c0 + I].y, pl)};
+            static_for<4>([&](auto I) {
+              if (I != j) y[I] = C{lane_read(v[RT - 1][I].x, pl), lane_read(v[RT - 1][I].y, pl)};
             });
           else
-            static_for<c1 - c0>([&](auto I) {
-              y[I] = C{lane_read(v[0][c0 + I].x, pl), lane_read(v[0][c0 + I].y, pl)};
+            static_for<4>([&](auto I) {
+              if (I != j) y[I] = C{lane_read(v[0][I].x, pl), lane_read(v[0][I].y, pl)};
             });
-          static_for<c1 - c0>([&](auto I) {
-            static_for<RT>([&](auto T) { v[T][c0 + I - 1] = fms_c(v[T][c0 + I], m[T], y[I]); });
+          static_for<RT>([&](auto T) {
+            static_for<3>([&](auto I) {  // the next column first
+              constexpr int c = (j + 1 + I) & 3;
+              v[T][c] = fms_c(v[T][c], m[T], y[c]);
+            });
+            // the column becomes Y's: -m below, U above and on the pivot row
+            const bool live = pos[T] > k;
+            v[T][j].x = live ? -m[T].x : v[T][j].x;
+            v[T][j].y = live ? -m[T].y : v[T][j].y;
           });
-        };
-        // the next column first: its search overlaps the other updates
-        update(std::integral_constant<int, 1>{}, std::integral_constant<int, 6>{});
-        search(k + 1);
-        update(std::integral_constant<int, 6>{}, std::integral_constant<int, 11>{});
-        update(std::integral_constant<int, 11>{}, std::integral_constant<int, 16>{});
-        static_for<RT>([&](auto T) { v[T][15] = fin[T]; });
-      }
-      if (l < kmax) {
-        s_perm[16 * P + l] = my_p;
-        s_uinv[16 * P + l] = my_inv;
-      }
-      if (sing && l == 0) s_sing = 1;
-      for (int j = kmax; j < 16; ++j)  // the register order after a narrow panel
+        });
+        if (sing && l == 0) s_sing = 1;
         static_for<RT>([&](auto T) {
-          const C first = v[T][0];
-          static_for<15>([&](auto Cc) { v[T][Cc] = v[T][Cc + 1]; });
-          v[T][15] = first;
+          const int r = l + 64 * T;
+          if (r < n) s_pos[r] = pos[T];
+          if (r < R) {
+            s_rowt[buf][r] = rowt[T];
+            static_for<4>([&](auto J) { pn[J * LD + r] = v[T][J]; });
+          }
         });
-      static_for<RT>([&](auto T) {
-        const int r = l + 64 * T;
-        if (r < n) s_pos[r] = pos[T];
-      });
-      if (P > 0) __syncthreads();  // the previous panel has been read
-      static_for<RT>([&](auto T) {
-        const int r = l + 64 * T;
-        if (r < R) {
-          s_rowt[r] = rowt[T];
-          static_for<16>([&](auto Cc) { pan[Cc * LD + r] = v[T][Cc]; });
-        }
-      });
-      __syncthreads();
-      static_for<NP>([&](auto S) {
-        static_for<4>([&](auto Q) {
-          const C x = pan[(4 * Q + lc) * LD + 16 * S + drow];
-          mr[S][Q] = x.x;
-          mi[S][Q] = x.y;
-        });
-      });
-    } else {
-      if (P > 0) __syncthreads();
+      }
+      // the panel is published; everyone has read the one before the last
       __syncthreads();
       // pivot rows of the wave's own columns -> scratch, row t = pivot step
-      if (kmax < 16) {
-        for (int e = l; e < 16 * 17; e += 64) scr[e] = C{0, 0};
+      if (kmax < 4) {
+        for (int e = l; e < 4 * 17; e += 64) scr[e] = C{0, 0};
         wave_lds_fence();
       }
       static_for<NP>([&](auto S) {
-        const int t = s_rowt[16 * S + drow];
-        if (t >= 0 && t < 16)
+        const int t = s_rowt[buf][16 * S + drow];
+        if (t >= 0 && t < 4)
           static_for<4>([&](auto Q) { scr[t * 17 + 4 * Q + lc] = C{mr[S][Q], mi[S][Q]}; });
       });
-      int rt[NP];
-      static_for<NP>([&](auto S) { rt[S] = s_rowt[16 * S + (l & 15)]; });
       wave_lds_fence();
-#pragma unroll 1
-      for (int kk = 0; kk < 4; ++kk) {
-        const int k = 4 * kk + la;
-        double br[4], bi[4];
-        static_for<4>([&](auto Q) {
-          const C x = scr[k * 17 + 4 * Q + lc];
-          br[Q] = x.x;
-          bi[Q] = x.y;
-        });
+      double br[4], bi[4];
+      static_for<4>([&](auto Q) {
+        const C x = scr[la * 17 + 4 * Q + lc];
+        br[Q] = x.x;
+        bi[Q] = x.y;
+      });
+      static_for<NP>([&](auto S) {
+        C z = pn[la * LD + 16 * S + (l & 15)];
+        if (la >= s_rowt[buf][16 * S + (l & 15)]) z = C{0, 0};
+        mfma_c4(z.x, z.y, br, bi, mr[S], mi[S]);
+        static_for<4>([&](auto Q) { pin(mr[S][Q]); pin(mi[S][Q]); });
+      });
+      if (w == P)  // the panel's own columns
         static_for<NP>([&](auto S) {
-          C z = pan[k * LD + 16 * S + (l & 15)];
-          if (k >= rt[S]) z = C{0, 0};
-          mfma_c4(z.x, z.y, br, bi, mr[S], mi[S]);
+          const C x = pn[lc * LD + 16 * S + drow];
+          mr[S][G] = x.x;
+          mi[S][G] = x.y;
         });
-      }
       wave_lds_fence();
-    }
+    });
   }
 
   // ---- rows into position order ----
@@ -813,7 +786,7 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
     fresh_lane();
     // U_ii X_i = Y_i row by row: row k of every column from the lanes holding it
 #pragma unroll 1
-    for (int k = 15; k >= 0; --k) {
+    for (int k = min(15, n - 1 - 16 * i); k >= 0; --k) {
       const int src = (16 * (k & 3) + 4 * (k >> 2) + lc) << 2;
       const C ui = s_uinv[16 * i + k];
       C t = C{0, 0};
@@ -836,8 +809,6 @@ __global__ __launch_bounds__(64 * NP, NP <= 3 ? 4 : NP <= 4 ? 3 : 2) void k_lu_i
         static_for<i>([&](auto S) {
           const C u = ub[((i * (i - 1)) / 2 + S) * 272 + col * 17 + row];
           mfma_c4(-u.x, -u.y, br, bi, mr[S], mi[S]);
-        });
-        static_for<i>([&](auto S) {
           static_for<4>([&](auto Q) { pin(mr[S][Q]); pin(mi[S][Q]); });
         });
       });
@@ -1219,12 +1190,18 @@ __global__ __launch_bounds__(NT) void k_inv_unperm(int n, const typename CT_<R>:
 
 // Largest order of the one-workgroup LU kernel, above it the blocked
 // Gauss-Jordan path.  1 / 500 / 2000 FP64 blocks, here against the thread-grid
-// LU kernel used before (us, launch and wait included): order 32 50 / 68 / 113
-// against 80 / 88 / 118, order 64 98 / 133 / 371 against 153 / 212 / 620, order
-// 96 214 / 439 / 1666 against 330 / 494 / 1702.  FP64 at order 128 the blocked
-// path is as fast (500: 0.70 against 0.84 ms, 5: 0.32 against 0.29) with smaller
-// residuals.  FP32 (the block computed in FP64): 200 blocks of order 128 take
-// 0.35 ms against 1.4 ms for Gauss-Jordan in LDS.
+// LU kernel used before (us, launch and wait included), at every batch no slower:
+//   order 17   34 /  38 /   65    51 /  55 /   69
+//   order 32   45 /  58 /   95    79 /  89 /  119
+//   order 48   67 /  89 /  206   118 / 160 /  461
+//   order 64   92 / 131 /  332   152 / 213 /  612
+//   order 65  122 / 241 /  874   199 / 276 /  958
+//   order 80  145 / 284 / 1049   241 / 332 / 1165
+//   order 96  189 / 380 / 1394   330 / 491 / 1697
+// FP64 at order 128 the blocked path is as fast (500: 0.70 against 0.84 ms, 5:
+// 0.32 against 0.29, with panels of 16 columns) with smaller residuals.  FP32
+// (the block computed in FP64): 200 blocks of order 128 take 0.35 ms against
+// 1.4 ms for Gauss-Jordan in LDS.
 template <typename R> constexpr int kLuMaxN = sizeof(R) == 8 ? 96 : 128;
 
 template <typename Kern>
