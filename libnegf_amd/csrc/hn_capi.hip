@@ -146,7 +146,7 @@ int inverse1(hipnegf_handle h, void *A, void *Ainv, size_t n) {
   hn::fill_int(status, 1, 0, s);
   hn::InvWork<R> w;
   void *wb = nullptr;
-  if ((int)n > hn::inv_lds_max_n(sizeof(R))) {
+  if ((int)n > hn::inv_wg_max_n(sizeof(R))) {
     HN_CHECK(hipMallocAsync(&wb, hn::inv_work_bytes((int)n, 1, sizeof(R)), s));
     w = hn::inv_work_carve<R>(wb, (int)n, 1);
   }
@@ -222,7 +222,7 @@ int inv_batched(hipnegf_engine e, int n, void *A, long long sA, void *Ainv, long
   hn::fill_int(dstatus, batch, 0, s);
   hn::InvWork<R> w;
   void *wb = nullptr;
-  if (n > hn::inv_lds_max_n(sizeof(R))) {
+  if (n > hn::inv_wg_max_n(sizeof(R))) {
     HN_CHECK(hipMalloc(&wb, hn::inv_work_bytes(n, batch, sizeof(R))));
     w = hn::inv_work_carve<R>(wb, n, batch);
   }
@@ -281,7 +281,7 @@ int inverse_noalloc(hipnegf_handle h, void *A, void *Ainv, size_t n) {
     throw std::runtime_error("hipnegf_Zinverse_noalloc: the current device is not the handle's");
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t bytes = n * n * sizeof(double2);
-  const bool blocked = (int)n > hn::inv_lds_max_n(8);
+  const bool blocked = (int)n > hn::inv_wg_max_n(8);
   const size_t need = al(bytes) + 256 + (blocked ? hn::inv_work_bytes((int)n, 1, 8) : 0);
   if (need > kScratchBytes) throw std::runtime_error("hipnegf_Zinverse_noalloc: scratch too small");
   char *base = (char *)scratch_ptr(cur);

@@ -295,7 +295,7 @@ void Engine::inverse(int n, double2 *A, long long sA, double2 *Ainv, long long s
   (void)precision;
   (void)o;
   InvWork<double> w;
-  if (n > inv_lds_max_n(8)) {
+  if (n > inv_wg_max_n(8)) {
     size_t mark = arena_.used;
     void *buf = arena_.take<char>(inv_work_bytes(n, batch, 8));
     w = inv_work_carve<double>(buf, n, batch);
@@ -963,7 +963,7 @@ void Engine::t_sweep_mixed(DevStruct &st, int B, const double *dE, const int *ds
   auto inv32 = [&](int n, float2 *A, float2 *Ainv) {
     InvWork<float> w;
     size_t m2 = arena_.used;
-    if (n > inv_lds_max_n(4)) w = inv_work_carve<float>(arena_.take<char>(inv_work_bytes(n, B, 4)), n, B);
+    if (n > inv_wg_max_n(4)) w = inv_work_carve<float>(arena_.take<char>(inv_work_bytes(n, B, 4)), n, B);
     inv_c(n, A, s2, Ainv, s2, B, nullptr, dstatus, w, stream_);
     arena_.used = m2;
   };

@@ -6,8 +6,8 @@ namespace hn {
 
 constexpr int kInvSuper = 64;  // max super-panel width: deferred rank-64 updates
 
-// Largest n handled by the one-workgroup LU kernel (no workspace needed).
-int inv_lds_max_n(int real_bytes);
+// Largest order inverted by one workgroup per block (no workspace needed).
+int inv_wg_max_n(int real_bytes);
 
 // Workspace of the blocked path, for `batch` items of order n.
 template <typename R>

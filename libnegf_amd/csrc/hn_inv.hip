@@ -5,7 +5,9 @@
 //
 // Blocks up to 96 (FP32: 128): one workgroup per block, LU with partial pivoting
 // and the substitutions in registers, on the matrix cores (k_lu_inv_mx; FP64 up
-// to 16 on a thread grid, k_lu_inv_2d).
+// to 16 on a thread grid, k_lu_inv_2d).  FP32 blocks of 129 to 140, the largest
+// that fit: Gauss-Jordan with partial pivoting in LDS, followed by the column
+// interchanges that undo the row pivoting (k_inv_lds).
 //
 // Large blocks (up to n = 1024): in-place Gauss-Jordan with lazy pivoting on
 // the row-major view M = A^T, so that rows of M are contiguous columns of A
@@ -29,6 +31,7 @@ namespace hn {
 namespace {
 
 constexpr int NT = 256;
+constexpr int kLdsBudget = 160 * 1024 - 2048;
 
 template <typename R> struct CT_;
 template <> struct CT_<double> { typedef double2 t; };
@@ -53,6 +56,98 @@ template <typename C> __device__ inline C crecip(C b) {
 }
 template <typename C> __device__ inline auto cabs1(C a) -> decltype(a.x) {
   return fabs(a.x) + fabs(a.y);
+}
+
+// wave-level argmax of (v, i): larger v wins, ties -> smaller index
+template <typename R> __device__ inline void wave_argmax(R &v, int &i) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    R ov = __shfl_xor(v, off);
+    int oi = __shfl_xor(i, off);
+    if (ov > v || (ov == v && oi >= 0 && (i < 0 || oi < i))) {
+      v = ov;
+      i = oi;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// single-workgroup LDS Gauss-Jordan (FP32 blocks of order 129 to 140)
+// ---------------------------------------------------------------------------
+template <typename R>
+__global__ __launch_bounds__(NT) void k_inv_lds(int n, typename CT_<R>::t *A, long long sA,
+                                                typename CT_<R>::t *Ainv, long long sAinv,
+                                                const int *active, int *status) {
+  typedef typename CT_<R>::t C;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (active && active[b] == 0) return;
+  C *M = (C *)smem;
+  C *rowbuf = M + (size_t)n * n;
+  C *colbuf = rowbuf + n;
+  int *perm = (int *)(colbuf + n);
+  __shared__ int s_p, s_sing;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const C *Ab = A + (long long)b * sA;
+  for (int e = tid; e < n * n; e += NT) M[e] = Ab[e];
+  if (tid == 0) s_sing = 0;
+  // 2-D thread mapping for the rank-1 update: thread -> (row i, column phase)
+  const int cpar = NT / n;  // n <= NT here
+  const int ui = tid % n, uj0 = tid / n;
+  const bool upd = uj0 < cpar;
+  __syncthreads();
+  for (int k = 0; k < n; ++k) {
+    if (wave == 0) {
+      R best = R(-1);
+      int bi = -1;
+      for (int i = k + lane; i < n; i += 64) {
+        R v = cabs1(M[i + (size_t)k * n]);
+        if (v > best) { best = v; bi = i; }
+      }
+      wave_argmax(best, bi);
+      if (lane == 0) {
+        s_p = bi < 0 ? k : bi;
+        if (!(best > R(0))) s_sing = 1;
+      }
+    }
+    __syncthreads();
+    const int p = s_p;
+    if (p != k)
+      for (int j = tid; j < n; j += NT) {
+        C t = M[k + (size_t)j * n];
+        M[k + (size_t)j * n] = M[p + (size_t)j * n];
+        M[p + (size_t)j * n] = t;
+      }
+    if (tid == 0) perm[k] = p;
+    __syncthreads();
+    const C pinv = crecip(M[k + (size_t)k * n]);
+    for (int j = tid; j < n; j += NT) rowbuf[j] = (j == k) ? pinv : cmul(M[k + (size_t)j * n], pinv);
+    for (int i = tid; i < n; i += NT) colbuf[i] = (i == k) ? C{0, 0} : M[i + (size_t)k * n];
+    __syncthreads();
+    if (upd) {
+      const C ci = colbuf[ui];
+      for (int j = uj0; j < n; j += cpar) {
+        size_t e = ui + (size_t)j * n;
+        if (ui == k) M[e] = rowbuf[j];
+        else if (j == k) M[e] = cneg(cmul(ci, pinv));
+        else M[e] = csub(M[e], cmul(ci, rowbuf[j]));
+      }
+    }
+    __syncthreads();
+  }
+  for (int k = n - 1; k >= 0; --k) {
+    const int p = perm[k];
+    if (p != k)
+      for (int i = tid; i < n; i += NT) {
+        C t = M[i + (size_t)k * n];
+        M[i + (size_t)k * n] = M[i + (size_t)p * n];
+        M[i + (size_t)p * n] = t;
+      }
+    __syncthreads();
+  }
+  C *Ob = Ainv + (long long)b * sAinv;
+  for (int e = tid; e < n * n; e += NT) Ob[e] = M[e];
+  if (tid == 0 && s_sing && status) atomicOr(&status[b], (int)ST_SINGULAR);
 }
 
 // ---------------------------------------------------------------------------
@@ -1204,6 +1299,19 @@ __global__ __launch_bounds__(NT) void k_inv_unperm(int n, const typename CT_<R>:
 // 1.4 ms for Gauss-Jordan in LDS.
 template <typename R> constexpr int kLuMaxN = sizeof(R) == 8 ? 96 : 128;
 
+// FP32 blocks above it that still fit in LDS (up to order 140) take Gauss-Jordan
+// there: residuals 1.0e-7, in the blocked FP32 path 1.5e-7 to 2.1e-7, though
+// that is 5 to 9 times faster (order 129, 1 block: 2.6 against 0.31 ms).
+template <typename R>
+size_t gj_lds_bytes(int n) {
+  typedef typename CT_<R>::t C;
+  return (size_t)n * n * sizeof(C) + 2 * (size_t)n * sizeof(C) + (size_t)n * sizeof(int);
+}
+template <typename R>
+bool gj_in_lds(int n) {
+  return sizeof(R) == 4 && n <= NT && gj_lds_bytes<R>(n) <= (size_t)kLdsBudget;
+}
+
 template <typename Kern>
 void allow_lds(Kern k, size_t bytes) {
   if (bytes > 64 * 1024)
@@ -1261,6 +1369,17 @@ void inv_impl(int n, typename CT_<R>::t *A, long long sA, typename CT_<R>::t *Ai
     lu_mx(n, A, sA, Ainv, sAinv, batch, active, status, s);
     return;
   }
+  if constexpr (sizeof(R) == 4) {
+    if (gj_in_lds<R>(n)) {
+      const size_t lds = gj_lds_bytes<R>(n);
+      allow_lds(k_inv_lds<R>, lds);
+      ProfScope ps(PT_INV_SMALL, sm_fl, sm_by, s);
+      hipLaunchKernelGGL(k_inv_lds<R>, dim3(batch), dim3(NT), lds, s, n, A, sA, Ainv, sAinv,
+                         active, status);
+      HN_CHECK(hipGetLastError());
+      return;
+    }
+  }
   if (n > 1024) throw std::runtime_error("inverse: block order > 1024 is not supported");
   if (sA < (long long)n * n || sAinv < (long long)n * n)
     throw std::runtime_error("inverse: item stride smaller than n*n");
@@ -1313,7 +1432,12 @@ void inv_impl(int n, typename CT_<R>::t *A, long long sA, typename CT_<R>::t *Ai
 
 }  // namespace
 
-int inv_lds_max_n(int real_bytes) { return real_bytes == 8 ? kLuMaxN<double> : kLuMaxN<float>; }
+int inv_wg_max_n(int real_bytes) {
+  if (real_bytes == 8) return kLuMaxN<double>;
+  int n = kLuMaxN<float>;
+  while (gj_in_lds<float>(n + 1)) ++n;
+  return n;
+}
 
 size_t inv_work_bytes(int n, int batch, int real_bytes) {
   size_t c = 2 * (size_t)real_bytes;

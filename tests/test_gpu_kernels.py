@@ -197,45 +197,75 @@ def test_gemm_tile_variants_bitwise(gpu, m, n, k, beta, ops):
     assert st["on"] and st["shapes"] >= 1
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 48, 49, 64, 65, 79, 96, 113, 127, 128])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 48, 49, 64, 65, 79, 96, 97, 100, 112, 113, 127, 128])
 def test_lu_inverse_many_blocks(gpu, n):
-    """The one-workgroup LU inverse over more blocks than one dispatch round
-    (the wave -> column rotation takes every value), with a singular block, a
-    block of equal magnitudes (pivot ties) and a NaN block among them: flags,
-    and residuals of the others at the backward error of LU with partial
-    pivoting, ||A X - I|| <= c n eps ||A|| ||X|| (c = 10 for growth)."""
+    """The one-workgroup LU inverse over enough blocks that the wave -> column
+    rotation (one step per 256 blocks, ceil(n/16) waves) takes every value, with
+    a singular block, a block of equal magnitudes (pivot ties) and a NaN block
+    among them: flags; blocks that repeat give bitwise the same inverse whatever
+    the rotation; and residuals of the others at the backward error of LU with
+    partial pivoting, ||A X - I|| <= c n eps ||A|| ||X|| (c = 10 for growth)."""
     torch, hip, eng = gpu
-    batch = 600
+    base = 200
+    rep = max(3, -(-(256 * (-(-n // 16) - 1) + 1) // base))
     g = torch.Generator(device="cuda").manual_seed(n)
-    A = torch.randn(batch, n, n, dtype=torch.complex128, device="cuda", generator=g)
+    A = torch.randn(base, n, n, dtype=torch.complex128, device="cuda", generator=g)
     A = A + A.mH + (0.2 + 1e-3j) * torch.eye(n, device="cuda")
     A[7, :, n // 2] = 0.0                                # a zero column: singular
     tie = torch.where(torch.rand(n, n, device="cuda", generator=g) < 0.5, 1.0, -1.0)
     A[11] = tie + n * 1j * torch.eye(n, device="cuda")   # |Re| + |Im| ties off the diagonal
     A[13, 0, n - 1] = complex(float("nan"), float("nan"))
-    X = torch.zeros_like(A)
-    st = torch.zeros(batch, dtype=torch.int32, device="cuda")
-    W = A.clone()
-    hip.check(hip.load().hipnegf_zinverse_batched(eng.handle, n, W.data_ptr(), n * n, X.data_ptr(), n * n,
-                                                  batch, st.data_ptr()))
-    s = st.cpu().numpy()
-    assert s[7] == 1 and (np.delete(s, [7, 13]) == 0).all()
-    assert not torch.isfinite(X[13].abs()).all()
-    ok = [b for b in range(batch) if b not in (7, 13)]
-    a, x = A[ok].cpu().numpy(), X[ok].cpu().numpy()
+    ok = [b for b in range(base) if b not in (7, 13)]
+
+    def run(f, W):
+        X = torch.zeros_like(W)
+        st = torch.zeros(len(W), dtype=torch.int32, device="cuda")
+        hip.check(f(eng.handle, n, W.data_ptr(), n * n, X.data_ptr(), n * n, len(W), st.data_ptr()))
+        X, s = X.view(rep, base, n, n), st.view(rep, base).cpu().numpy()
+        assert (X[:, ok] == X[:1, ok]).all()
+        assert not torch.isfinite(X[:, 13].abs()).flatten(1).all(1).any()
+        assert (s[:, 7] == 1).all() and (s[:, ok] == 0).all()
+        return X[0, ok].cpu().numpy(), s
+
+    x, _ = run(hip.load().hipnegf_zinverse_batched, A.repeat(rep, 1, 1))
+    a = A[ok].cpu().numpy()
     res = np.linalg.norm(a @ x - np.eye(n), axis=(1, 2))
     bound = 10 * n * 2.2e-16 * np.linalg.norm(a, axis=(1, 2)) * np.linalg.norm(x, axis=(1, 2))
     assert (res <= bound).all(), (res / bound).max()
     # complex FP32 in and out: the FP64 inverse of the rounded block, rounded once
-    Wc = A.to(torch.complex64)
-    Xc = torch.zeros_like(Wc)
-    hip.check(hip.load().hipnegf_cinverse_batched(eng.handle, n, Wc.data_ptr(), n * n, Xc.data_ptr(), n * n,
-                                                  batch, st.data_ptr()))
-    ac, xc = A.to(torch.complex64)[ok].cpu().numpy().astype(np.complex128), Xc[ok].cpu().numpy()
+    xc, s = run(hip.load().hipnegf_cinverse_batched, A.to(torch.complex64).repeat(rep, 1, 1))
+    assert (s[:, 13] == 1).all()
+    ac = A.to(torch.complex64)[ok].cpu().numpy().astype(np.complex128)
     ref = np.linalg.inv(ac)
     cond = np.linalg.norm(ac, axis=(1, 2)) * np.linalg.norm(ref, axis=(1, 2))
     err = np.abs(xc - ref).max(axis=(1, 2)) / np.abs(ref).max(axis=(1, 2))
     assert (err <= 1.2e-7 + 10 * n * 2.2e-16 * cond).all()
+
+
+@pytest.mark.parametrize("n", [129, 136, 140, 141])
+def test_cinverse_above_lu(gpu, n):
+    """FP32 blocks above the LU kernel: up to order 140 (the largest that fits)
+    Gauss-Jordan in LDS, whose residuals measure 1.0e-7 ||A|| ||X|| where the
+    blocked path's measure 1.5e-7 to 2.1e-7; singular and NaN blocks flagged."""
+    torch, hip, eng = gpu
+    g = torch.Generator(device="cuda").manual_seed(n)
+    H = torch.randn(42, n, n, dtype=torch.complex128, device="cuda", generator=g)
+    A = (0.3 + 1e-3j) * torch.eye(n, device="cuda") - (H + H.mH) / 2
+    A[40, :, 5] = 0.0
+    A[41, n - 1, 0] = complex(float("nan"), 0.0)
+    A = A.to(torch.complex64)
+    W, X = A.clone(), torch.zeros_like(A)
+    st = torch.zeros(42, dtype=torch.int32, device="cuda")
+    hip.check(hip.load().hipnegf_cinverse_batched(eng.handle, n, W.data_ptr(), n * n, X.data_ptr(), n * n, 42,
+                                                  st.data_ptr()))
+    s = st.cpu().numpy()
+    a, x = A[:40].cpu().numpy().astype(np.complex128), X[:40].cpu().numpy().astype(np.complex128)
+    nrm = lambda d: np.linalg.norm(d, axis=(1, 2))
+    res = nrm(a @ x - np.eye(n)) / (nrm(a) * nrm(x))
+    assert (s[:41] == [0] * 40 + [1]).all()
+    assert res.mean() <= (1.25e-7 if n <= 140 else 2.5e-7), res.mean()
+    if n <= 140:
+        assert s[41] == 1 and not torch.isfinite(X[41].abs()).all()
 
 
 @pytest.mark.parametrize("n", [1, 16, 17, 40, 64, 65, 96, 97, 128])
