@@ -276,8 +276,8 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// (key, pos) pair reduction over G consecutive lanes (G = 4, 8 or 16): the
-// larger key wins, equal keys go to the smaller pos
+// (key, pos) pair reduction over 8 consecutive lanes: the larger key wins, equal
+// keys go to the smaller pos
 template <int CTRL> __device__ inline void best_dpp(unsigned long long &k, int &p) {
   const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(k >> 32), CTRL, 0xF, 0xF, false);
   const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)k, CTRL, 0xF, 0xF, false);
@@ -288,11 +288,10 @@ template <int CTRL> __device__ inline void best_dpp(unsigned long long &k, int &
     p = op;
   }
 }
-template <int G> __device__ inline void group_best(unsigned long long &k, int &p) {
-  best_dpp<0xB1>(k, p);                  // quad_perm [1,0,3,2]
-  best_dpp<0x4E>(k, p);                  // quad_perm [2,3,0,1]
-  if (G >= 8) best_dpp<0x141>(k, p);     // row_half_mirror
-  if (G >= 16) best_dpp<0x140>(k, p);    // row_mirror
+__device__ inline void group_best8(unsigned long long &k, int &p) {
+  best_dpp<0xB1>(k, p);   // quad_perm [1,0,3,2]
+  best_dpp<0x4E>(k, p);   // quad_perm [2,3,0,1]
+  best_dpp<0x141>(k, p);  // row_half_mirror
 }
 // x - m y with the FMA order of the elimination updates
 __device__ inline double2 fms_c(double2 x, double2 m, double2 y) {
@@ -338,14 +337,13 @@ __device__ __forceinline__ double2 pick0(const double2 (&v)[TB][TB], int r) {
 // The thread column owning column col (register column JJ) publishes it:
 // pivoted rows' entries into the triangular U array, unpivoted rows' into
 // colbuf (the next multipliers), and the pivot's row, position and
-// reciprocal.  Called by every thread; only the owner's wave works.
+// reciprocal.
 template <int G, int TB, int JJ>
 __device__ __forceinline__ void lu_publish(int col, int tid, const LuBlk<TB> &B, double2 *Ut,
                                            double2 *colbuf, int *s_perm, int *s_pospiv,
                                            double2 *s_uinv, int *s_sing) {
   const int cb = tid / G, rb = tid % G;
   const int oc = col / TB;
-  if ((tid >> 6) != (oc * G) >> 6) return;  // wave-uniform: only the owner's wave
   unsigned long long key = 0, kk[TB];
   int bp = 0x7fffffff;
   static_for<TB>([&](auto I) {
@@ -362,7 +360,7 @@ __device__ __forceinline__ void lu_publish(int col, int tid, const LuBlk<TB> &B,
       bp = B.pos[i];
     }
   });
-  group_best<G>(key, bp);
+  group_best8(key, bp);
   if (cb == oc) {
     static_for<TB>([&](auto I) {
       constexpr int i = I;
@@ -384,7 +382,7 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
                                                      int *__restrict__ status) {
   typedef double2 C;
   constexpr int LD = G * TB;  // rows (and columns) of the padded block
-  static_assert(G * G >= 64 || G * G == 16, "thread columns inside one wave");
+  static_assert(G == 8, "one wave, thread columns of 8 lanes");
   const int b = blockIdx.x;
   if (active && active[b] == 0) return;
   extern __shared__ __align__(16) unsigned char lsm[];
@@ -1330,8 +1328,9 @@ void launch_lu(int n, IO *A, long long sA, IO *Ainv, long long sAinv, int batch,
 template <typename IO>
 void lu_mx(int n, IO *A, long long sA, IO *Ainv, long long sAinv, int batch, const int *active,
            int *status, hipStream_t s) {
+  if constexpr (sizeof(IO) == sizeof(float2))  // FP64 up to 16: k_lu_inv_2d
+    if (n <= 16) return launch_lu<1>(n, A, sA, Ainv, sAinv, batch, active, status, s);
   switch ((n + 15) / 16) {
-    case 1: return launch_lu<1>(n, A, sA, Ainv, sAinv, batch, active, status, s);
     case 2: return launch_lu<2>(n, A, sA, Ainv, sAinv, batch, active, status, s);
     case 3: return launch_lu<3>(n, A, sA, Ainv, sAinv, batch, active, status, s);
     case 4: return launch_lu<4>(n, A, sA, Ainv, sAinv, batch, active, status, s);
@@ -1358,7 +1357,7 @@ void inv_impl(int n, typename CT_<R>::t *A, long long sA, typename CT_<R>::t *Ai
   if (n <= kLuMaxN<R>) {
     ProfScope ps(PT_INV_SMALL, sm_fl, sm_by, s);
     if constexpr (sizeof(R) == 8) {
-      if (n <= 16) {  // one wave either way: 2000 blocks of order 10 take 32 us here, 37 below
+      if (n <= 16) {  // one wave either way: 2000 blocks of order 10 take 32 us here, 36 below
         const size_t lds = std::max<size_t>(1, (size_t)n * (n - 1) / 2) * sizeof(double2);
         hipLaunchKernelGGL((k_lu_inv_2d<8, 2>), dim3(batch), dim3(64), lds, s, n, A, sA, Ainv, sAinv,
                            active, status);

@@ -136,7 +136,9 @@ def check(rc: int):
 # launch-timing tags (hipnegf_profile_*)
 PT_GEMM_MASKED, PT_GEMM_SWEEP, PT_GEMM_INV, PT_INV_PANEL, PT_INV_SMALL, PT_FUSED = range(6)
 # Kernel serving each tag for FP64 blocks with K, N >= 128 (the 64 x 128 tiling);
-# smaller GEMMs of a tag run on k_gemm<double, tag>.
+# smaller GEMMs of a tag run on k_gemm<double, tag>.  One-workgroup inverses are
+# k_lu_inv_mx's but for FP64 up to order 16 (k_lu_inv_2d) and FP32 of order 129
+# to 140 (k_inv_lds).
 PT_NAMES = {PT_GEMM_MASKED: "k_gemm_w<0>", PT_GEMM_SWEEP: "k_gemm_w<1>",
             PT_GEMM_INV: "k_gemm_w<2>", PT_INV_PANEL: "k_inv_gj",
             PT_INV_SMALL: "k_lu_inv_mx", PT_FUSED: "k_t_fused"}
