@@ -4,8 +4,9 @@
 // For principal layers of up to kFusedMaxN orbitals every block fits in LDS
 // many times over, and the batched engine's cost is launches and host polls
 // (one launch per block operation per step, one convergence poll per
-// decimation iteration).  Here one wave per item runs, without leaving the
-// kernel: each contact's Sancho-Rubio decimation with its own convergence
+// decimation iteration).  Here one workgroup per item (one wave, or one per
+// contact while the items are few) runs, without leaving the kernel: each
+// contact's Sancho-Rubio decimation with its own convergence
 // test (contselfenergy.F90:271-340; both stopping rules), the self-energy
 // Sigma = Tlc GS Tcl (:445-491, 552-566), the backward sweep at real E
 // (build_ESH, iterative.F90:1956-1982; calculate_gsmr_blocks,
@@ -366,11 +367,13 @@ bool Engine::t_fused(DevStruct &st, int nitems, const double *dE, const int *dsl
   auto lds_of = [&](int W) {
     return (size_t)fused_mats(W) * n * n * sizeof(double2) + (size_t)W * 64 * sizeof(int);
   };
-  // Two waves per item while all items are resident at once (256 CUs of 160 KiB
-  // LDS): the call then takes one item's chain (200 items of 20 layers, order 10:
-  // 1.83 -> 1.23 ms; order 16: 3.98 -> 2.57).  Beyond that the LDS per item
-  // decides, twelve blocks against twenty-two (order 16, 500 items: 4.1 ms with
-  // one wave each).
+  // Two waves per item while the LDS of 256 CUs (160 KiB each) holds all items,
+  // from order 6 on the call then takes one item's chain; one wave each against
+  // two, ten layers: order 16, 256 items 3.79 / 2.14 ms, 300 items 3.89 / 4.16;
+  // order 10, 1024 items 1.87 / 1.19 ms, 2000 items 2.49 / 2.54.  Up to order 5
+  // the registers (12 workgroups of two waves per CU) hold fewer items than the
+  // LDS, and two waves are the faster ones still: order 5, 4096 items 1.50 / 1.22
+  // ms, order 2, 8000 items 1.08 / 0.93.
   const long long fit2 = 256LL * (long long)((160 * 1024 - 1024) / (lds_of(2) + 256));
   const bool two = nitems <= fit2;
   {

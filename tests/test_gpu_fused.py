@@ -1,5 +1,6 @@
-"""The fused small-block transmission (one launch per call, one wave per (E,k)
-item running both decimations, the sweep and the trace; hn_fused.hip) against
+"""The fused small-block transmission (one launch per call, one workgroup per
+(E,k) item running both decimations, the sweep and the trace, with two waves
+where all items are resident at once and one wave beyond; hn_fused.hip) against
 the oracle and against the batched block-operation path (HIPNEGF_NO_FUSED)."""
 import numpy as np
 import pytest
@@ -91,3 +92,23 @@ def test_disordered_ribbon_fused_vs_batched(gpu):
     bar = np.maximum(1e-10, 4 * sp)
     big = Tref > 1e-6 * Tref.max()
     assert ((np.abs(T - Tref) / Tref)[big] <= bar[big] + 1e-10).all()
+
+
+@pytest.mark.parametrize("n,nitems", [(16, 257), (16, 300), (12, 800), (10, 1100), (7, 2400), (5, 4400)])
+def test_one_wave_and_two_waves_bitwise(gpu, n, nitems):
+    """More items than the two-wave limit (256 CUs times the 1, 3, 4, 9 or 17
+    workgroups whose LDS fits) run one wave per item: T, counts and status to
+    the bit those of sub-calls small enough for two waves, whose accuracy the
+    tests above hold; a sample of the counts against the oracle."""
+    hip, eng = gpu
+    s = wl.ribbon(n, 5, disorder=0.4, seed=n)
+    E = np.linspace(-3.1, 3.1, nitems)
+    ds = hip.DeviceStructure(s)
+    T, ncyc, st = hip.solve_transmission(eng, ds, E, delta=1e-5)
+    assert (st == 0).all()
+    for a in range(0, nitems, 200):
+        Tp, np_, sp = hip.solve_transmission(eng, ds, E[a:a + 200], delta=1e-5)
+        assert np.array_equal(Tp, T[a:a + 200]) and np.array_equal(np_, ncyc[a:a + 200])
+        assert np.array_equal(sp, st[a:a + 200])
+    pick = np.arange(3, nitems, max(1, nitems // 12))
+    assert np.array_equal(ncyc[pick], _oracle(s, E[pick], 1e-5)[1])
