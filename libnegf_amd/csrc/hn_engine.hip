@@ -2042,15 +2042,13 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
   double2 *Gam = arena_.take<double2>(SB * std::max(ncont, 1));
   for (int c = 0; c < ncont; ++c) gamma_batched(Sig + c * SB, s2, Gam + c * SB, s2, n, B, stream_);
 
-  // with inelastic stores covering exactly this batch, G^r and the diagonal
-  // G^n blocks are formed in the stores themselves (same [block][item] layout)
-  const bool in_store = io && io->i0 == 0 && io->NI == B;
+  // with inelastic stores, G^r and G^n are formed in the stores themselves
+  // (cache_Gr, cache_Gn; masked launches leave converged items' blocks as they
+  // were); without, only their diagonal blocks are kept
   double2 *g = arena_.take<double2>(SB * nbl);
-  double2 *Grd = in_store ? io->G[0] : arena_.take<double2>(SB * nbl);
-  double2 *Gru = in_store ? io->G[1] : arena_.take<double2>(SB * std::max(nbl - 1, 1));
-  double2 *Grl = in_store ? io->G[2] : arena_.take<double2>(SB * std::max(nbl - 1, 1));
+  double2 *Grd_list = io ? nullptr : arena_.take<double2>(SB * nbl);
   double2 *Sn = arena_.take<double2>(SB * nbl);
-  double2 *Gnd = in_store ? io->G[3] : arena_.take<double2>(SB * nbl);
+  double2 *Gnd_list = io ? nullptr : arena_.take<double2>(SB * nbl);
   double2 *Gnd_old = arena_.take<double2>(SB * nbl);
   const bool s_general = (st.smode & S_OFFDIAG) != 0;
   double2 *Gnu_old = s_general ? arena_.take<double2>(SB * std::max(nbl - 1, 1)) : nullptr;
@@ -2083,6 +2081,8 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
   const int frm_stride = so.frm_per_item ? ncont + 1 : 0;
   const double2 one = Z(1), zero = Z(0), mone = Z(-1);
   auto blk = [&](double2 *base, int i) { return base + (long long)i * SB; };
+  auto Grd = [&](int i) { return io ? ost(0, i) : blk(Grd_list, i); };
+  auto Gnd = [&](int i) { return io ? ost(3, i) : blk(Gnd_list, i); };
 
   auto form_diag = [&](int i, double2 *out) {
     FormArgs f;
@@ -2148,18 +2148,19 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
       mm(Uc, OP_N, blk(g, 1), OP_N, Ug, one, zero);
       mm(Ug, OP_N, Lc, OP_N, D, mone, one);
     }
-    inverse(n, D, s2, blk(Grd, 0), s2, B, act, dstatus, PREC_FP64, o, n_active);
+    inverse(n, D, s2, Grd(0), s2, B, act, dstatus, PREC_FP64, o, n_active);
     // ---- Gr tridiagonal blocks, i = 2..nbl (1-based) ----
     for (int i = 1; i < nbl; ++i) {
       mm(blk(g, i), OP_N, blk(Lc, i - 1), OP_N, blk(gL, i - 1), one, zero);
-      mm(blk(gL, i - 1), OP_N, blk(Grd, i - 1), OP_N, blk(Grl, i - 1), mone, zero);
-      mm(blk(Grd, i - 1), OP_N, blk(Ug, i - 1), OP_N, blk(Gru, i - 1), mone, zero);
-      copy_batched(blk(Grd, i), s2, blk(g, i), s2, s2, B, act, stream_);
-      mm(blk(Grl, i - 1), OP_N, blk(Ug, i - 1), OP_N, blk(Grd, i), mone, one);
+      double2 *Grl = io ? ost(2, i - 1) : W2;
+      mm(blk(gL, i - 1), OP_N, Grd(i - 1), OP_N, Grl, mone, zero);
+      if (io) mm(Grd(i - 1), OP_N, blk(Ug, i - 1), OP_N, ost(1, i - 1), mone, zero);
+      copy_batched(Grd(i), s2, blk(g, i), s2, s2, B, act, stream_);
+      mm(Grl, OP_N, blk(Ug, i - 1), OP_N, Grd(i), mone, one);
     }
     // ---- set_Gr: sigma_r = c^2 diag(Gr) ----
     for (int i = 0; i < nbl; ++i)
-      diag_extract_masked(blk(Grd, i), s2, n, B, sig_r + (long long)i * n, ndev, c2 + (long long)i * n,
+      diag_extract_masked(Grd(i), s2, n, B, sig_r + (long long)i * n, ndev, c2 + (long long)i * n,
                           act, stream_);
     // ---- Sigma_n(i,i) = diag(sigma_n) + contact terms ----
     for (int i = 0; i < nbl; ++i) {
@@ -2191,28 +2192,28 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
       mm(W1, OP_N, ug, OP_C, blk(Sn, i), one, one);
     }
     // ---- Gn(1,1) = Gr(1,1) Sigma_n(1,1) Gr(1,1)^H ----
-    mm(blk(Sn, 0), OP_N, blk(Grd, 0), OP_C, W1, one, zero);
-    mm(blk(Grd, 0), OP_N, W1, OP_N, blk(Gnd, 0), one, zero);
+    mm(blk(Sn, 0), OP_N, Grd(0), OP_C, W1, one, zero);
+    mm(Grd(0), OP_N, W1, OP_N, Gnd(0), one, zero);
     fill_int(reinterpret_cast<int *>(err), 2 * B, 0, stream_);
     // ---- downward recursion ----
     for (int i = 0; i + 1 < nbl; ++i) {
-      // with inelastic stores, Gn(i+1,i) / Gn(i,i+1) are formed in them directly
-      // (cache_Gn; masked launches leave converged items' blocks as they were)
       double2 *Gnl_i = io ? ost(5, i) : Gnl, *Gnu_i = io ? ost(4, i) : Gnu;
+      double2 *Gru = io ? ost(1, i) : W1;
+      if (!io) mm(Grd(i), OP_N, blk(Ug, i), OP_N, Gru, mone, zero);
       // Gn(i+1,i) = g Sn(i+1) Gr(i,i+1)^H + g Sigma_n(i+1,i) Gr(i,i)^H - g L Gn(i,i)
       mm(blk(g, i + 1), OP_N, blk(Sn, i + 1), OP_N, gSn, one, zero);
-      mm(gSn, OP_N, blk(Gru, i), OP_C, Gnl_i, one, zero);
+      mm(gSn, OP_N, Gru, OP_C, Gnl_i, one, zero);
       if (inel_off) {
         mm(blk(g, i + 1), OP_N, ist(4, i), OP_C, W2, one, zero);
-        mm(W2, OP_N, blk(Grd, i), OP_C, Gnl_i, one, one);
+        mm(W2, OP_N, Grd(i), OP_C, Gnl_i, one, one);
       }
-      mm(blk(gL, i), OP_N, blk(Gnd, i), OP_N, Gnl_i, mone, one);
+      mm(blk(gL, i), OP_N, Gnd(i), OP_N, Gnl_i, mone, one);
       // Gn(i,i+1) = Gn(i+1,i)^H is formed only where it is kept or tested
       if (io || s_general) dagger_batched(Gnl_i, s2, Gnu_i, s2, n, n, B, act, stream_);
       // Gn(i+1,i+1), the same with Gr(i+1,i+1), Gr(i+1,i) and Gn(i,i+1)
-      mm(gSn, OP_N, blk(Grd, i + 1), OP_C, blk(Gnd, i + 1), one, zero);
-      if (inel_off) mm(W2, OP_N, blk(Grl, i), OP_C, blk(Gnd, i + 1), one, one);
-      mm(blk(gL, i), OP_N, Gnl_i, OP_C, blk(Gnd, i + 1), mone, one);
+      mm(gSn, OP_N, Grd(i + 1), OP_C, Gnd(i + 1), one, zero);
+      if (inel_off) mm(W2, OP_N, ost(2, i), OP_C, Gnd(i + 1), one, one);
+      mm(blk(gL, i), OP_N, Gnl_i, OP_C, Gnd(i + 1), mone, one);
       if (s_general) {  // off-diagonal S entries enter the convergence test
         // Gn(i+1,i) = Gn(i,i+1)^H, so |dGn(i+1,i)(r,c)| = |dGn(i,i+1)(c,r)|: one pass over
         // Gn(i,i+1) with the union of the S(i,i+1) pattern and the transposed S(i+1,i) pattern
@@ -2222,35 +2223,25 @@ void Engine::scba_batch(DevStruct &st, int B, const double *dE, const int *dslot
     }
     // ---- set_Gn and the convergence test ----
     for (int i = 0; i < nbl; ++i) {
-      diag_extract_masked(blk(Gnd, i), s2, n, B, sig_n + (long long)i * n, ndev, c2 + (long long)i * n,
+      diag_extract_masked(Gnd(i), s2, n, B, sig_n + (long long)i * n, ndev, c2 + (long long)i * n,
                           act, stream_);
-      masked_diff(blk(Gnd, i), blk(Gnd_old, i), s2, n, n, sd ? 1 : 0, sd ? st.ref(BK_SD, i) : BlkRef(),
+      masked_diff(Gnd(i), blk(Gnd_old, i), s2, n, n, sd ? 1 : 0, sd ? st.ref(BK_SD, i) : BlkRef(),
                   BlkRef(), dslot, err, act, B, stream_);
     }
     scba_state(err, so.tol, pass, so.niter, act, diters, derr, B, stream_);
   }
-  // ---- cache_Gr / cache_Gn for the inelastic model (each item's last pass) ----
-  if (io && !in_store)
-    for (int i = 0; i < nbl; ++i) {
-      copy_batched(ost(0, i), s2, blk(Grd, i), s2, s2, B, nullptr, stream_);
-      copy_batched(ost(3, i), s2, blk(Gnd, i), s2, s2, B, nullptr, stream_);
-      if (i + 1 < nbl) {
-        copy_batched(ost(1, i), s2, blk(Gru, i), s2, s2, B, nullptr, stream_);
-        copy_batched(ost(2, i), s2, blk(Grl, i), s2, s2, B, nullptr, stream_);
-      }
-    }
   // ---- Meir-Wingreen current per contact ----
   for (int c = 0; c < ncont; ++c) {
     const int b = st.cblk[c] - 1;
-    trace_mw(Gam + c * SB, blk(Gnd, b), blk(Grd, b), s2, n, so.frm, frm_stride, c, ncont, B, dcurr,
+    trace_mw(Gam + c * SB, Gnd(b), Grd(b), s2, n, so.frm, frm_stride, c, ncont, B, dcurr,
              stream_);
   }
   if (gn_diag)
     for (int i = 0; i < nbl; ++i)
-      diag_extract_masked(blk(Gnd, i), s2, n, B, gn_diag + (long long)i * n, ndev, nullptr, nullptr, stream_);
+      diag_extract_masked(Gnd(i), s2, n, B, gn_diag + (long long)i * n, ndev, nullptr, nullptr, stream_);
   if (gr_diag)
     for (int i = 0; i < nbl; ++i)
-      diag_extract_masked(blk(Grd, i), s2, n, B, gr_diag + (long long)i * n, ndev, nullptr, nullptr, stream_);
+      diag_extract_masked(Grd(i), s2, n, B, gr_diag + (long long)i * n, ndev, nullptr, nullptr, stream_);
   // per-item status: contacts | inverses
   {
     std::vector<int> hs((size_t)B * ncont), hst(B);
@@ -2273,9 +2264,10 @@ void Engine::scba_mw(DevStruct &st, int nitems, const double *dE, const int *dsl
   // n: the (uniform) PL order; nm >= n also covers contact surface blocks
   const int n = st.bsz[0], nm = st.nmax(), nbl = st.nbl;
   const size_t b2 = (size_t)nm * nm * sizeof(double2);
-  // G^r/G^n block lists, ESH off-diagonal blocks and kept products (13 nbl) + sweep temporaries (8) + contact decimation and
-  // self-energy workspace (12 per contact) + inverse workspace + per-orbital vectors
-  const size_t per_item = b2 * (size_t)(13 * nbl + 12 * st.ncont + 16) +
+  // G^r/G^n block lists, ESH off-diagonal blocks and kept products (at most 10 nbl, 11
+  // budgeted) + sweep temporaries (8) + contact decimation and self-energy workspace
+  // (12 per contact) + inverse workspace + per-orbital vectors
+  const size_t per_item = b2 * (size_t)(11 * nbl + 12 * st.ncont + 16) +
                           inv_work_bytes(nm, std::max(st.ncont, 1), 8) + (size_t)n * nbl * 48 + 1024;
   const int B = pick_batch(st, nitems, o, per_item);
   last_batch_ = B;
@@ -2426,7 +2418,7 @@ void Engine::inel_mw(DevStruct &st, const double *E, const double *frm, const So
   // batch of the elastic sweeps (same per-item budget as scba_mw)
   const int nm = st.nmax();
   const size_t b2 = (size_t)nm * nm * sizeof(double2);
-  const size_t per_item = b2 * (size_t)(13 * nbl + 12 * ncont + 16) +
+  const size_t per_item = b2 * (size_t)(11 * nbl + 12 * ncont + 16) +
                           inv_work_bytes(nm, ncont, 8) + (size_t)n * nbl * 48 + 1024;
   const int B = pick_batch(st, (int)std::min<long long>(NI, 1 << 30), o, per_item);
   last_batch_ = B;

@@ -158,3 +158,26 @@ def test_scba_batch_invariance(gpu):
                                max_batch=mb, lanes=lanes)
         np.testing.assert_array_equal(r0["curr"], r1["curr"])
         np.testing.assert_array_equal(r0["iters"], r1["iters"])
+
+
+def test_scba_workspace(gpu):
+    """One item's workspace, as the device memory the call leaves with the
+    engine: 11 blocks per layer, 12 per contact and 16 more, plus 5 % for the
+    inverse's workspace and the per-orbital vectors.  Memory a structure needs
+    beyond that it would be refused for."""
+    import torch
+    hip, _ = gpu
+    n, nbl = 256, 60
+    s = wl.ribbon(n, nbl, disorder=0.2, seed=3)
+    tiny = hip.DeviceStructure(wl.ribbon(n, 2, disorder=0.2, seed=3))
+    ds = hip.DeviceStructure(s)
+    eng = hip.Engine(0)
+    run = lambda d, nb: hip.solve_scba_mw(eng, d, np.array([0.3]), np.full(n * nb, 0.05), 1, 1e-8,
+                                          [1.0, 0.0, 0.0], 3, delta=1e-4, max_batch=1)
+    run(tiny, 2)                                       # kernels loaded
+    held = (11 * 2 + 12 * 2 + 16) * n * n * 16
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    assert (run(ds, nbl)["status"] == 0).all()
+    used = before - torch.cuda.mem_get_info()[0] + held
+    assert used <= 1.05 * (11 * nbl + 12 * 2 + 16) * n * n * 16, used
