@@ -512,8 +512,8 @@ __global__ __launch_bounds__(G * G) void k_lu_inv_2d(int n, const double2 *__res
 // 2.4 - 2.9 times LAPACK's error, four give 0.95 - 0.99, and the transmission of
 // ribbons of 24 to 90 orbitals had 4 - 22 % more error in the mean over 800
 // energies than elimination one column at a time, now 4 % more to 6 % less.  And
-// since four columns take 16 registers per row of a lane, so that two workgroups
-// of 5 or 6 waves share a CU.
+// since four columns take 16 registers per row of a lane instead of 64, so that
+// more waves share a SIMD.
 //
 // Then every wave sorts its rows by position and the back substitution
 // U X = Y runs by blocks of 16: U_ii X_i = Y_i row by row (explicit U_ii^-1 lost
@@ -629,8 +629,13 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// waves per SIMD the registers are kept for: whole workgroups of NP waves
-constexpr int lu_waves(int np) { return np <= 4 ? 4 : np <= 6 ? 3 : 2; }
+// Waves per SIMD the registers are kept for.  Workgroups of 5 waves need 4: with
+// 3 (no spills) the second workgroup of a CU found no room on the SIMD that
+// holds two waves of the first; order 65, 1 / 500 / 2000 blocks 122 / 241 / 874
+// us with 3, 128 / 181 / 708 with 4.  Of 6 waves 3: LDS and 263 spilled registers
+// eat up what the second workgroup gives (order 96, 189 / 376 / 1394 us with 3,
+// 222 / 337 / 1387 with 4).
+constexpr int lu_waves(int np) { return np <= 5 ? 4 : np <= 6 ? 3 : 2; }
 
 template <int NP, typename IO>
 __global__ __launch_bounds__(64 * NP, lu_waves(NP)) void k_lu_inv_mx(int n, const IO *__restrict__ A,
@@ -1288,13 +1293,16 @@ __global__ __launch_bounds__(NT) void k_inv_unperm(int n, const typename CT_<R>:
 //   order 32   45 /  58 /   95    79 /  89 /  119
 //   order 48   67 /  89 /  206   118 / 160 /  461
 //   order 64   92 / 131 /  332   152 / 213 /  612
-//   order 65  122 / 241 /  874   199 / 276 /  958
-//   order 80  145 / 284 / 1049   241 / 332 / 1165
+//   order 65  128 / 181 /  708   199 / 276 /  958
+//   order 80  151 / 218 /  847   241 / 332 / 1165
 //   order 96  189 / 380 / 1394   330 / 491 / 1697
 // FP64 at order 128 the blocked path is as fast (500: 0.70 against 0.84 ms, 5:
 // 0.32 against 0.29, with panels of 16 columns) with smaller residuals.  FP32
-// (the block computed in FP64): 200 blocks of order 128 take 0.35 ms against
-// 1.4 ms for Gauss-Jordan in LDS.
+// (the block computed in FP64), 1 / 2000 blocks against Gauss-Jordan in LDS: order
+// 64 93 / 321 against 260 / 676 us, order 65 134 / 721 against 314 / 790, order 128
+// 0.28 / 2.2 against 1.4 / 11.3 ms; with one row or column beyond a multiple of 16
+// and 2000 blocks it is 9 % slower at orders 17 and 33 (63 against 58 us, 147
+// against 135), where one block takes 34 against 46 us and 53 against 88.
 template <typename R> constexpr int kLuMaxN = sizeof(R) == 8 ? 96 : 128;
 
 // FP32 blocks above it that still fit in LDS (up to order 140) take Gauss-Jordan
