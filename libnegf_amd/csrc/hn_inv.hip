@@ -1296,8 +1296,10 @@ __global__ __launch_bounds__(NT) void k_inv_unperm(int n, const typename CT_<R>:
 //   order 65  128 / 181 /  708   199 / 276 /  958
 //   order 80  151 / 218 /  847   241 / 332 / 1165
 //   order 96  189 / 380 / 1394   330 / 491 / 1697
-// FP64 at order 128 the blocked path is as fast (500: 0.70 against 0.84 ms, 5:
-// 0.32 against 0.29, with panels of 16 columns) with smaller residuals.  FP32
+// FP64 orders 97 to 128 stay on the blocked path, whose residuals are up to 15 %
+// smaller (2.4e-16 ||A|| ||X||, here 2.4e-16 to 2.8e-16), though it takes longer:
+// order 97 229 / 646 / 2635 us against 213 / 434 / 1660 here, order 128 292 / 831 /
+// 3376 against 294 / 615 / 2346.  FP32
 // (the block computed in FP64), 1 / 2000 blocks against Gauss-Jordan in LDS: order
 // 64 93 / 321 against 260 / 676 us, order 65 134 / 721 against 314 / 790, order 128
 // 0.28 / 2.2 against 1.4 / 11.3 ms; with one row or column beyond a multiple of 16
